@@ -113,8 +113,7 @@ int choose_launch(Context *ctx, uint32_t B, uint32_t n_bases, size_t extra_lds, 
   *bases_in_lds = bases_bytes <= 32 * 1024;
   if (!*bases_in_lds) bases_bytes = 0;
   bases_bytes += extra_lds;  // camera records
-  // the short stack: per level and lane a block address, its Child field (u32 each) and its
-  // chunk (u16)
+  // the short stack: per level and lane a block's Child field and chunk (u32 each)
   const auto stack_bytes = [&](uint32_t n) { return ((size_t)n * wg * kStackEntryBytes + 15) & ~(size_t)15; };
   while (levels > 1 && bases_bytes + stack_bytes(levels) > lds_limit) levels--;
   if (bases_bytes + stack_bytes(levels) > lds_limit)

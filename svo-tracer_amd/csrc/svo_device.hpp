@@ -223,6 +223,87 @@ __device__ __forceinline__ uint32_t compare_canon(uint32_t depth, uint64_t px, u
   return depth > k ? depth - k : 1u;
 }
 
+// ---- fast steps (the fused trace kernel) ----
+// An ordinary cone's direction: every component is 0 or of a magnitude in [2^-60, 2^20) (finite,
+// with a finite reciprocal), one of them not 0.  When no axis of such a cone stands on the face it
+// moves towards, the distances to the boundary are 1..2^62, the least a = |distance * inverse| is
+// finite, and the move along a minor axis n, |d_n * inv_m| * distance_m, is at most
+// distance_n (1 + 6 * 2^-24): below 2^-1 of the cube, so it neither saturates nor is NaN.
+__device__ __forceinline__ bool ordinary_component(float d) {
+  const uint32_t e = __float_as_uint(d) & 0x7fffffffu;
+  return e == 0u || (e >= (67u << 23) && e < (147u << 23));
+}
+__device__ __forceinline__ bool ordinary_directions(float dx, float dy, float dz) {
+  return ordinary_component(dx) && ordinary_component(dy) && ordinary_component(dz) &&
+         (dx != 0.0f || dy != 0.0f || dz != 0.0f);
+}
+// A camera whose cone footprint is its FoV times the distance: no depth of field (the footprint
+// is then max(FoV * m, 0)), finite position and FoV.
+__device__ __forceinline__ bool ordinary_camera(const float o[3], float fov, float dof0) {
+  return fabsf(o[0]) < 1048576.0f && fabsf(o[1]) < 1048576.0f && fabsf(o[2]) < 1048576.0f && fov >= 0.0f &&
+         fov < 1048576.0f && dof0 == 0.0f;
+}
+// 2^32 times the origin's coordinate along the canonical axis (c grows from the face moved towards).
+__device__ __forceinline__ float canon_origin(float o, bool pos) { return (pos ? 1.0f - o : o) * 4294967296.0f; }
+
+// The footprint decides nothing but comparisons with powers of two.  Computed from the high words
+// (m = distance * 2^32) it differs from cone_at's by less than 2^-22.2 of the cube in the distance
+// (2^-24 from the origin, 2^-25 from each conversion, over three axes) and a few ulp after: less
+// than 2^-15.9 of it at distances of 2^-6 and more.  Unsure: nearer than that, or within 2^-14 of
+// a power of two; then cone_at decides.
+__device__ __forceinline__ bool cone_unsure(float m, float cone) {
+  return m < 67108864.0f || ((__float_as_uint(cone) + 0x200u) & 0x7fffffu) < 0x400u;
+}
+
+// A 64-bit distance as 2^-32 times its correctly rounded float (1 <= d < 2^63): the top 32
+// significant bits with the rest as a sticky bit, converted once.
+__device__ __forceinline__ float distance32(uint32_t hi, uint32_t lo) {
+  const uint32_t n = hi ? (uint32_t)__builtin_clz(hi) : 32u;
+  const uint64_t t = (((uint64_t)hi << 32) | lo) << n;
+  uint32_t sticky;  // min(low word, 1), which the compiler turns into a comparison and a select
+  asm("v_min_u32 %0, 1, %1" : "=v"(sticky) : "v"((uint32_t)t));
+  const float f = (float)((uint32_t)(t >> 32) | sticky);
+  return __builtin_amdgcn_ldexpf(f, -(int)n);
+}
+
+// A move of y (in units of 2^-32, 0 <= y < 2^31) as a 64-bit fixed-point number, truncated: the
+// fraction of y is exact, and so is its scaling.
+__device__ __forceinline__ uint64_t move64(float y) {
+  const uint32_t hi = (uint32_t)y;
+  const uint32_t lo = (uint32_t)(__builtin_amdgcn_fractf(y) * 4294967296.0f);
+  return ((uint64_t)hi << 32) | lo;
+}
+
+// traverse_canon for an ordinary cone on levels 1..30 (lv = 31 - level): the same values, from the
+// high words where the level's mask ends in them.  An axis that reaches its face is left at 0 or
+// one past it (ULONG_MAX, which traverse_canon pins to 0); returns whether any did.
+__device__ __forceinline__ bool traverse_fast(uint32_t lv, uint64_t &cx, uint64_t &cy, uint64_t &cz, float dx, float dy,
+                                              float dz, float ix, float iy, float iz, uint32_t signs) {
+  const uint32_t hm = (1u << lv) - 1u;
+  const auto round = [&](uint64_t c, bool pos) -> uint64_t {
+    const uint32_t h = (uint32_t)(c >> 32);
+    uint32_t carry;
+    const uint32_t lo = __builtin_addc((uint32_t)c, 0u, (pos || h > hm) ? 1u : 0u, &carry);
+    return ((uint64_t)((h & hm) + carry) << 32) | lo;
+  };
+  const uint64_t d0 = round(cx, signs & 1u), d1 = round(cy, signs & 2u), d2 = round(cz, signs & 4u);
+  const float f0 = distance32((uint32_t)(d0 >> 32), (uint32_t)d0), f1 = distance32((uint32_t)(d1 >> 32), (uint32_t)d1),
+              f2 = distance32((uint32_t)(d2 >> 32), (uint32_t)d2);
+  const float a0 = fabsf(f0 * ix), a1 = fabsf(f1 * iy), a2 = fabsf(f2 * iz);
+  const float least = fminf(fminf(a0, a1), a2);
+  const bool m0 = a0 == least, m1 = !m0 && a1 == least;
+  const float inv_m = m0 ? ix : (m1 ? iy : iz), f_m = m0 ? f0 : (m1 ? f1 : f2);
+  const uint64_t na = move64(fabsf(((m0 ? dy : dx) * inv_m) * f_m));
+  const uint64_t nb = move64(fabsf(((m0 || m1 ? dz : dy) * inv_m) * f_m));
+  const uint64_t n0 = m0 ? d0 : na;
+  const uint64_t n1 = m1 ? d1 : (m0 ? na : nb);
+  const uint64_t n2 = (m0 || m1) ? nb : d2;
+  cx -= n0;
+  cy -= n1;
+  cz -= n2;
+  return cx + 1ull <= 1ull || cy + 1ull <= 1ull || cz + 1ull <= 1ull;
+}
+
 // Morton code of the top `depth` bits (depth <= 10) from the high words of the positions.
 __device__ __forceinline__ uint32_t morton_top_hi(uint32_t depth, uint32_t xh, uint32_t yh, uint32_t zh) {
   const uint32_t s = 32u - depth;

@@ -11,9 +11,8 @@ namespace svo {
 
 // work counters sit on separate 128-byte lines (u32 stride)
 constexpr uint32_t kCounterStride = 32;
-// LDS bytes per short-stack entry of the trace kernel: block address and Child (u32 each),
-// chunk (u16)
-constexpr uint32_t kStackEntryBytes = 10;
+// LDS bytes per short-stack entry of the trace kernel: a block's Child and chunk (u32 each)
+constexpr uint32_t kStackEntryBytes = 8;
 // Most slots of the trace kernel's per-workgroup LDS table of usage groups already ticked in
 // the launch (direct-mapped on the group index, u32 each); a launch uses a power of two up to
 // this many, or none, so that the table never lowers the work-groups a CU holds
