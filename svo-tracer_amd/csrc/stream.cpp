@@ -13,6 +13,7 @@
 #include <algorithm>
 #include <cstring>
 #include <string>
+#include <vector>
 
 #include "svo_internal.hpp"
 #include "svo_runtime.hpp"
@@ -485,21 +486,46 @@ extern "C" int svo_stream_update(svo_context *ctx, const svo_terrain *t, const s
 
 namespace {
 
+// A piece of the build's device memory.
+struct Piece {
+  void *ptr = nullptr;
+  size_t bytes = 0;
+};
+
 struct BuildLevel {
   uint32_t n = 0;      // nodes (dense level: x-outer positions, 8^(B+2))
   uint32_t n_int = 0;  // nodes that get children
-  std::shared_ptr<DeviceBuffer> flag, irank, cells, alloc, writes, rank, start, post;
+  Piece flag, irank, cells, alloc, writes, rank, start, post;
 };
 
+// The build's temporaries are carved from a few slabs, each four times the last one's size (up to
+// 512 MiB) or what the piece needs, all released at the end: some fifty allocations and as many
+// frees of a depth-12 build (70 and 180 us each) took as long as its kernels.
 struct Builder {
   Context *ctx;
   hipStream_t s;
-  std::vector<std::shared_ptr<DeviceBuffer>> keep;
+  std::vector<std::shared_ptr<DeviceBuffer>> slabs;
+  size_t used = 0, next = (size_t)32 << 20;
 
-  int buf(size_t bytes, std::shared_ptr<DeviceBuffer> *out) { return new_buffer(std::max<size_t>(bytes, 4), out); }
+  int buf(size_t bytes, Piece *out) {
+    bytes = (std::max<size_t>(bytes, 4) + 255) & ~(size_t)255;
+    if (slabs.empty() || bytes > slabs.back()->bytes - used) {
+      std::shared_ptr<DeviceBuffer> slab;
+      int rc = new_buffer(std::max(bytes, next), &slab);
+      if (rc && bytes < next) rc = new_buffer(bytes, &slab);
+      if (rc) return rc;
+      slabs.push_back(slab);
+      used = 0;
+      next = std::min(4 * next, (size_t)512 << 20);
+    }
+    out->ptr = (char *)slabs.back()->ptr + used;
+    out->bytes = bytes;
+    used += bytes;
+    return SVO_OK;
+  }
   template <class T>
-  T *ptr(const std::shared_ptr<DeviceBuffer> &b) {
-    return b ? (T *)b->ptr : nullptr;
+  T *ptr(const Piece &b) {
+    return (T *)b.ptr;
   }
   int launched(int r, const char *what) {
     return r ? fail(SVO_ERR_HIP, std::string("svo_terrain_build_tree: launch ") + what) : SVO_OK;
@@ -509,9 +535,9 @@ struct Builder {
     if (e == hipSuccess) e = hipStreamSynchronize(s);
     return e == hipSuccess ? SVO_OK : hip_fail(e, "svo_terrain_build_tree: read back");
   }
-  // Exclusive ranks of a 0/1 flag array and the number of ones.
-  int rank(const uint32_t *flags, uint32_t n, std::shared_ptr<DeviceBuffer> *out, uint32_t *total) {
-    std::shared_ptr<DeviceBuffer> counts;
+  // Exclusive ranks of a flag array (bit 0) and the number of ones.
+  int rank(const uint32_t *flags, uint32_t n, Piece *out, uint32_t *total) {
+    Piece counts;
     int rc = buf(((size_t)n / 1024 + 2) * 4, &counts);
     if (!rc) rc = buf((size_t)n * 4, out);
     if (rc) return rc;
@@ -523,8 +549,8 @@ struct Builder {
     *total = 0;
     return n ? read(c + chunks, total, 4) : SVO_OK;
   }
-  int fill(const std::shared_ptr<DeviceBuffer> &b, int byte) {
-    hipError_t e = hipMemsetAsync(b->ptr, byte, b->bytes, s);
+  int fill(void *p, int byte, size_t bytes) {
+    hipError_t e = hipMemsetAsync(p, byte, bytes, s);
     return e == hipSuccess ? SVO_OK : hip_fail(e, "svo_terrain_build_tree: clear");
   }
 };
@@ -546,13 +572,16 @@ int build_tree_device(Context *ctx, const GeomView &g, uint32_t base_depth, uint
 
   // Bases, and the level-(B+1) cells: mixed ones in PopulateInitialBlocks' write order,
   // empty ones (ascending) as the head of the free-group FIFO
-  std::shared_ptr<DeviceBuffer> bases, mixed, empty, mixed_rank, empty_rank, empties;
-  if ((rc = bd.buf((size_t)pow_sum(B) * 2, &bases)) || (rc = bd.buf((size_t)dense_groups * 4, &mixed)) ||
-      (rc = bd.buf((size_t)dense_groups * 4, &empty)))
+  std::shared_ptr<DeviceBuffer> bases_out;
+  if ((rc = new_buffer((size_t)pow_sum(B) * 2, &bases_out))) return rc;
+  uint16_t *bases = (uint16_t *)bases_out->ptr;
+  Piece mixed, empty, mixed_rank, empty_rank, empties, last;
+  if ((rc = bd.buf((size_t)dense_groups * 4, &mixed)) || (rc = bd.buf((size_t)dense_groups * 4, &empty)) ||
+      (rc = bd.buf(4, &last)) || (rc = bd.fill(last.ptr, 0, 4)))
     return rc;
-  if ((rc = bd.launched(launch_bt_bases(g, bd.ptr<uint16_t>(bases), B, bd.s), "bases"))) return rc;
-  if ((rc = bd.launched(launch_bt_octant_flags(bd.ptr<uint16_t>(bases), B, bd.ptr<uint32_t>(mixed),
-                                               bd.ptr<uint32_t>(empty), bd.s),
+  if ((rc = bd.launched(launch_bt_bases(g, bases, B, bd.s), "bases"))) return rc;
+  if ((rc = bd.launched(launch_bt_octant_flags(bases, B, bd.ptr<uint32_t>(mixed), bd.ptr<uint32_t>(empty),
+                                               bd.ptr<uint32_t>(last), bd.s),
                         "octants")))
     return rc;
   uint32_t n_mixed = 0, n_empties = 0;
@@ -570,7 +599,7 @@ int build_tree_device(Context *ctx, const GeomView &g, uint32_t base_depth, uint
   std::vector<BuildLevel> lv(1);
   lv[0].n = n0;
   if ((rc = bd.buf((size_t)n0 * 4, &lv[0].flag))) return rc;
-  if ((rc = bd.launched(launch_bt_dense_flags(g, bd.ptr<uint16_t>(bases), B, max_depth,
+  if ((rc = bd.launched(launch_bt_dense_flags(g, bases, B, max_depth,
                                               bd.ptr<uint32_t>(lv[0].flag), bd.s),
                         "dense flags")))
     return rc;
@@ -587,9 +616,12 @@ int build_tree_device(Context *ctx, const GeomView &g, uint32_t base_depth, uint
     if (n > 0xffffffffull) return fail(SVO_ERR_CAPACITY, "svo_terrain_build_tree: a level above 2^32 blocks");
     BuildLevel c;
     c.n = (uint32_t)n;
+    if (L >= max_depth) {  // the deepest level: childless
+      lv.push_back(c);
+      break;
+    }
     if ((rc = bd.buf((size_t)n * 4, &c.flag))) return rc;
-    if ((rc = bd.launched(launch_bt_level_flags(g, bd.ptr<uint3>(p.cells), c.n, L, max_depth,
-                                                bd.ptr<uint32_t>(c.flag), bd.s),
+    if ((rc = bd.launched(launch_bt_level_flags(g, bd.ptr<uint3>(p.cells), c.n, L, bd.ptr<uint32_t>(c.flag), bd.s),
                           "level flags")))
       return rc;
     if ((rc = bd.rank(bd.ptr<uint32_t>(c.flag), c.n, &c.irank, &c.n_int))) return rc;
@@ -598,14 +630,14 @@ int build_tree_device(Context *ctx, const GeomView &g, uint32_t base_depth, uint
                                                 bd.ptr<uint32_t>(c.irank), c.n, bd.ptr<uint3>(c.cells), bd.s),
                           "level cells")))
       return rc;
-    lv.push_back(std::move(c));
+    lv.push_back(c);
   }
 
   // bottom-up: groups and block writes under every internal block
   for (size_t i = lv.size(); i-- > 0;) {
     BuildLevel &l = lv[i];
     if ((rc = bd.buf((size_t)l.n_int * 4, &l.alloc)) || (rc = bd.buf((size_t)l.n_int * 4, &l.writes))) return rc;
-    const BuildLevel *c = i + 1 < lv.size() ? &lv[i + 1] : nullptr;
+    const BuildLevel *c = i + 1 < lv.size() && lv[i + 1].flag.ptr ? &lv[i + 1] : nullptr;
     if ((rc = bd.launched(launch_bt_sizes(l.n_int, c ? bd.ptr<uint32_t>(c->flag) : nullptr,
                                           c ? bd.ptr<uint32_t>(c->irank) : nullptr,
                                           c ? bd.ptr<uint32_t>(c->alloc) : nullptr,
@@ -616,7 +648,7 @@ int build_tree_device(Context *ctx, const GeomView &g, uint32_t base_depth, uint
   }
   // top-down: pre-order ranks (FIFO entries) and write positions; the dense level's
   // internal blocks are the roots, in x-outer / z-inner order
-  std::shared_ptr<DeviceBuffer> totals;
+  Piece totals;
   if ((rc = bd.buf(16, &totals))) return rc;
   uint32_t *tot = bd.ptr<uint32_t>(totals);
   if ((rc = bd.buf((size_t)lv[0].n_int * 4, &lv[0].rank)) || (rc = bd.buf((size_t)lv[0].n_int * 4, &lv[0].start)))
@@ -640,6 +672,7 @@ int build_tree_device(Context *ctx, const GeomView &g, uint32_t base_depth, uint
   }
   for (size_t i = 0; i + 1 < lv.size(); i++) {
     BuildLevel &l = lv[i], &c = lv[i + 1];
+    if (!c.flag.ptr) break;  // the deepest level's blocks need neither
     if ((rc = bd.buf((size_t)c.n_int * 4, &c.rank)) || (rc = bd.buf((size_t)c.n_int * 4, &c.start)) ||
         (rc = bd.buf((size_t)c.n * 4, &c.post)))
       return rc;
@@ -657,28 +690,30 @@ int build_tree_device(Context *ctx, const GeomView &g, uint32_t base_depth, uint
   const uint64_t groups64 = dense_groups + (taken > n_empties ? taken - n_empties : 0);
   if (groups64 * 8 > 0xffffffffull) return fail(SVO_ERR_CAPACITY, "svo_terrain_build_tree: more than 2^32 blocks");
   const uint32_t n_groups = (uint32_t)groups64;
-  std::shared_ptr<DeviceBuffer> blocks, post, gparent, maxes;
-  if ((rc = bd.buf((size_t)n_groups * 128, &blocks)) || (rc = bd.buf((size_t)n_groups * 32, &post)) ||
-      (rc = bd.buf((size_t)n_groups * 4, &gparent)) || (rc = bd.buf(16, &maxes)))
+  std::shared_ptr<DeviceBuffer> blocks;
+  Piece post, gparent;
+  if ((rc = new_buffer((size_t)n_groups * 128, &blocks)) || (rc = bd.buf((size_t)n_groups * 32, &post)) ||
+      (rc = bd.buf((size_t)n_groups * 4, &gparent)))
     return rc;
-  if ((rc = bd.fill(blocks, 0)) || (rc = bd.fill(post, 0xff)) || (rc = bd.fill(gparent, 0xff)) ||
-      (rc = bd.fill(maxes, 0)))
+  // only the dense groups can stay unwritten: every other group in use is a FIFO entry that was
+  // taken, with a parent and eight blocks
+  if ((rc = bd.fill(blocks->ptr, 0, (size_t)dense_groups * 128)) ||
+      (rc = bd.fill(post.ptr, 0xff, (size_t)dense_groups * 32)) ||
+      (rc = bd.fill(gparent.ptr, 0xff, (size_t)dense_groups * 4)))
     return rc;
   GroupFifo fifo{bd.ptr<uint32_t>(empties), n_empties, dense_groups, capacity};
-  BuildOut o{bd.ptr<uint4>(blocks), bd.ptr<uint32_t>(post), bd.ptr<uint32_t>(gparent),
-             bd.ptr<unsigned long long>(maxes)};
-  if ((rc = bd.launched(launch_bt_write_dense(g, bd.ptr<uint16_t>(bases), B, bd.ptr<uint32_t>(lv[0].flag),
+  BuildOut o{(uint4 *)blocks->ptr, bd.ptr<uint32_t>(post), bd.ptr<uint32_t>(gparent)};
+  if ((rc = bd.launched(launch_bt_write_dense(g, bases, B, bd.ptr<uint32_t>(lv[0].flag),
                                               bd.ptr<uint32_t>(lv[0].irank), bd.ptr<uint32_t>(lv[0].rank),
-                                              bd.ptr<uint32_t>(mixed_rank), fifo, o, bd.s),
+                                              bd.ptr<uint32_t>(mixed_rank), L0 < max_depth, fifo, o, bd.s),
                         "write dense")))
     return rc;
   for (size_t i = 1; i < lv.size(); i++) {
     const BuildLevel &p = lv[i - 1], &c = lv[i];
-    const bool deeper = i + 1 < lv.size() || c.n_int;
-    if ((rc = bd.launched(launch_bt_write_level(g, bd.ptr<uint3>(p.cells), bd.ptr<uint32_t>(p.rank), c.n,
-                                                L0 + (uint32_t)i, deeper ? bd.ptr<uint32_t>(c.flag) : nullptr,
-                                                bd.ptr<uint32_t>(c.irank), bd.ptr<uint32_t>(c.rank),
-                                                bd.ptr<uint32_t>(c.post), fifo, o, bd.s),
+    if ((rc = bd.launched(launch_bt_write_level(g, bd.ptr<uint3>(p.cells), bd.ptr<uint32_t>(p.rank),
+                                                bd.ptr<uint32_t>(p.start), c.n, L0 + (uint32_t)i,
+                                                bd.ptr<uint32_t>(c.flag), bd.ptr<uint32_t>(c.irank),
+                                                bd.ptr<uint32_t>(c.rank), bd.ptr<uint32_t>(c.post), fifo, o, bd.s),
                           "write level")))
       return rc;
   }
@@ -690,9 +725,16 @@ int build_tree_device(Context *ctx, const GeomView &g, uint32_t base_depth, uint
   // (writes above everything written before) that ends at M: the first record of the run
   // sets count = a + 1, the next (a + 1) finds count equal to it and leaves it, the next
   // sets it again, and so on.
-  unsigned long long mx[2] = {0, 0};
-  if ((rc = bd.read(bd.ptr<unsigned long long>(maxes), mx, 16))) return rc;
-  const uint32_t M = (uint32_t)mx[0], M1 = (uint32_t)mx[1];
+  // M1, the dense level's largest address, ends the last mixed cell; the DFS writes fill the groups
+  // of the FIFO entries taken, whose largest is the last one taken.
+  uint32_t last_mixed = 0, top_group = 0;
+  if ((rc = bd.read(last.ptr, &last_mixed, 4))) return rc;
+  if (taken > n_empties)
+    top_group = n_groups - 1;
+  else if (taken && (rc = bd.read(bd.ptr<uint32_t>(empties) + (taken - 1), &top_group, 4)))
+    return rc;
+  const uint32_t M1 = last_mixed ? 8 * last_mixed - 1 : 0u;
+  const uint32_t M = std::max(M1, taken ? 8 * top_group + 7 : 0u);
   uint32_t count = n_mixed ? M1 + 1 : 0u;  // nothing is written without a mixed level-(B+1) cell
   if (n_mixed && M > M1) {
     // records among the DFS writes: a is one when every written address above it was
@@ -724,15 +766,16 @@ int build_tree_device(Context *ctx, const GeomView &g, uint32_t base_depth, uint
   }
   if (block_count) *block_count = count;
 
-  // outputs: the context's Bases / Blocks (/ Usages) and, if asked, a host tree
+  // outputs: the context's Bases / Blocks (/ Usages) and, if asked, a host tree.  The blocks are
+  // bound where they were written (the allocation ends with the last group in use, the buffer with
+  // the last block counted).
   const uint32_t out_groups = (count + 7) / 8;
-  std::shared_ptr<DeviceBuffer> cb, ck;
-  if ((rc = new_buffer((size_t)pow_sum(B) * 2, &cb)) || (rc = new_buffer((size_t)count * 16, &ck))) return rc;
-  cb->flags = SVO_BUFFER_READ_ONLY;
-  ck->flags = SVO_BUFFER_READ_ONLY;
-  hipError_t e = hipMemcpyAsync(cb->ptr, bases->ptr, cb->bytes, hipMemcpyDeviceToDevice, bd.s);
-  if (e == hipSuccess && count) e = hipMemcpyAsync(ck->ptr, blocks->ptr, ck->bytes, hipMemcpyDeviceToDevice, bd.s);
-  if (e != hipSuccess) return hip_fail(e, "svo_terrain_build_tree: copy");
+  if (count)
+    blocks->bytes = (size_t)count * 16;
+  else if ((rc = new_buffer(0, &blocks)))
+    return rc;
+  bases_out->flags = SVO_BUFFER_READ_ONLY;
+  blocks->flags = SVO_BUFFER_READ_ONLY;
   std::shared_ptr<DeviceBuffer> cu;
   if (with_usages) {
     if ((rc = new_buffer((size_t)out_groups * sizeof(svo_usage), &cu))) return rc;
@@ -750,15 +793,15 @@ int build_tree_device(Context *ctx, const GeomView &g, uint32_t base_depth, uint
     tree->t.bases.resize(pow_sum(B));
     tree->t.blocks.resize(count);
     tree->t.group_parent.resize(out_groups);
-    if ((rc = bd.read(bases->ptr, tree->t.bases.data(), tree->t.bases.size() * 2))) return rc;
+    if ((rc = bd.read(bases, tree->t.bases.data(), tree->t.bases.size() * 2))) return rc;
     if (count && (rc = bd.read(blocks->ptr, tree->t.blocks.data(), (size_t)count * 16))) return rc;
-    if (out_groups && (rc = bd.read(gparent->ptr, tree->t.group_parent.data(), (size_t)out_groups * 4))) return rc;
+    if (out_groups && (rc = bd.read(gparent.ptr, tree->t.group_parent.data(), (size_t)out_groups * 4))) return rc;
     *out = tree.release();
   }
-  e = hipStreamSynchronize(bd.s);
+  hipError_t e = hipStreamSynchronize(bd.s);
   if (e != hipSuccess) return hip_fail(e, "svo_terrain_build_tree");
-  ctx->buffers[SVO_BUF_BASES] = cb;
-  ctx->buffers[SVO_BUF_BLOCKS] = ck;
+  ctx->buffers[SVO_BUF_BASES] = bases_out;
+  ctx->buffers[SVO_BUF_BLOCKS] = blocks;
   if (cu) ctx->buffers[SVO_BUF_USAGES] = cu;
   ctx->tree_max_depth = max_depth;
   return SVO_OK;

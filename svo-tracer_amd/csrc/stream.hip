@@ -47,9 +47,9 @@ __device__ uint16_t make_chunk(const TerrainView &t, uint32_t level, uint32_t x,
   return chunk;
 }
 
-// MakeBlock, TreeBuilder.cs:74-93 (ColourB takes colour[1] and ColourG colour[2], as there).
-__device__ uint4 make_block(const TerrainView &t, uint32_t level, uint32_t x, uint32_t y, uint32_t z) {
-  const uint16_t chunk = make_chunk(t, level, x, y, z);
+// MakeBlock, TreeBuilder.cs:74-93 (ColourB takes colour[1] and ColourG colour[2], as there), of the
+// cell's chunk.
+__device__ uint4 make_block(const TerrainView &t, uint32_t level, uint32_t x, uint32_t y, uint32_t z, uint32_t chunk) {
   float lo, hi;
   footprint(t, level, x, y, &lo, &hi);
   int16_t pitch, yaw;
@@ -57,7 +57,7 @@ __device__ uint4 make_block(const TerrainView &t, uint32_t level, uint32_t x, ui
   terrain::attributes(t.spec, t.top, level, x, y, z, hi, &pitch, &yaw, rgb);
   uint4 b;
   b.x = kU32Max;
-  b.y = (uint32_t)chunk | ((uint32_t)(uint16_t)pitch << 16);
+  b.y = chunk | ((uint32_t)(uint16_t)pitch << 16);
   // yaw @8, R @10, G @11 (= rgb[2]), B @12 (= rgb[1]), opacity @13 = 255, spare, gloss 0
   b.z = (uint32_t)(uint16_t)yaw | ((uint32_t)rgb[0] << 16) | ((uint32_t)rgb[2] << 24);
   b.w = (uint32_t)rgb[1] | (255u << 8);
@@ -96,6 +96,11 @@ __device__ void geom_classify(const GeomView &g, uint32_t level, uint32_t x, uin
 }
 
 __device__ uint16_t geom_chunk(const GeomView &g, uint32_t level, uint32_t x, uint32_t y, uint32_t z) {
+  if (g.kind == SVO_GEOMETRY_SPHERE_NOISE) {
+    double sdf[14];
+    shapes::noise_points<true, false>(g.noise, level, x, y, z, sdf);
+    return (uint16_t)shapes::noise_chunk(g.noise, level, sdf);
+  }
   uint16_t chunk = 0;
   for (uint32_t k = 0; k < 8; k++) {
     bool a, e;
@@ -106,18 +111,31 @@ __device__ uint16_t geom_chunk(const GeomView &g, uint32_t level, uint32_t x, ui
   return chunk;
 }
 
-__device__ uint4 geom_block(const GeomView &g, uint32_t level, uint32_t x, uint32_t y, uint32_t z) {
-  if (g.kind == SVO_GEOMETRY_FBM_HEIGHTFIELD) return make_block(g.t, level, x, y, z);
-  const uint16_t chunk = geom_chunk(g, level, x, y, z);
+// known: `chunk` is the cell's chunk already; otherwise it is made here.
+__device__ uint4 geom_block(const GeomView &g, uint32_t level, uint32_t x, uint32_t y, uint32_t z, bool known,
+                            uint32_t chunk) {
+  if (g.kind == SVO_GEOMETRY_FBM_HEIGHTFIELD)
+    return make_block(g.t, level, x, y, z, known ? chunk : (uint32_t)make_chunk(g.t, level, x, y, z));
   int16_t pitch = 0, yaw = 0;
   uint8_t rgb[3] = {255, 255, 255};  // boxes: white, no normal
-  if (g.kind == SVO_GEOMETRY_SPHERES)
-    shapes::spheres_attributes(g.shapes, g.count, shapes::cell_box(level, x, y, z), &pitch, &yaw, rgb);
-  else if (g.kind != SVO_GEOMETRY_CUBES)
-    shapes::noise_attributes(g.noise, level, x, y, z, &pitch, &yaw, rgb);
+  if (g.kind == SVO_GEOMETRY_SPHERE_NOISE) {
+    double sdf[14];
+    if (known) {
+      shapes::noise_points<false, true>(g.noise, level, x, y, z, sdf);
+    } else {
+      shapes::noise_points<true, true>(g.noise, level, x, y, z, sdf);
+      chunk = shapes::noise_chunk(g.noise, level, sdf);
+    }
+    terrain::normal_angle(sdf[8] - sdf[9], sdf[10] - sdf[11], sdf[12] - sdf[13], &pitch, &yaw);
+    shapes::noise_colour(g.noise, level, x, y, z, rgb);
+  } else {
+    if (!known) chunk = geom_chunk(g, level, x, y, z);
+    if (g.kind == SVO_GEOMETRY_SPHERES)
+      shapes::spheres_attributes(g.shapes, g.count, shapes::cell_box(level, x, y, z), &pitch, &yaw, rgb);
+  }
   uint4 b;
   b.x = kU32Max;
-  b.y = (uint32_t)chunk | ((uint32_t)(uint16_t)pitch << 16);
+  b.y = chunk | ((uint32_t)(uint16_t)pitch << 16);
   b.z = (uint32_t)(uint16_t)yaw | ((uint32_t)rgb[0] << 16) | ((uint32_t)rgb[2] << 24);
   b.w = (uint32_t)rgb[1] | (255u << 8);
   return b;
@@ -165,7 +183,8 @@ __global__ __launch_bounds__(kWg) void seed_dense_kernel(TerrainView t, const ui
     const uint32_t bp = la >> 3;  // the level-(B+1) cell
     uint4 b = make_uint4(0u, 0u, 0u, 0u);
     if (((bases[base_start + (bp >> 3)] >> ((bp & 7u) * 2)) & 3u) == 3u)
-      b = make_block(t, level, compact3(la), compact3(la >> 1), compact3(la >> 2));
+      b = make_block(t, level, compact3(la), compact3(la >> 1), compact3(la >> 2),
+                     make_chunk(t, level, compact3(la), compact3(la >> 1), compact3(la >> 2)));
     blocks[la] = b;
   }
 }
@@ -269,7 +288,8 @@ __global__ __launch_bounds__(kWg) void brick_kernel(TerrainView t, RequestSource
   const uint32_t D = r.depth, s = 64u - D;
   const uint32_t x = (uint32_t)(r.location[0] >> s), y = (uint32_t)(r.location[1] >> s),
                  z = (uint32_t)(r.location[2] >> s);
-  bricks[8ull * k + c] = make_block(t, D + 1u, 2 * x + (c & 1u), 2 * y + ((c >> 1) & 1u), 2 * z + ((c >> 2) & 1u));
+  const uint32_t bx = 2 * x + (c & 1u), by = 2 * y + ((c >> 1) & 1u), bz = 2 * z + ((c >> 2) & 1u);
+  bricks[8ull * k + c] = make_block(t, D + 1u, bx, by, bz, make_chunk(t, D + 1u, bx, by, bz));
   if (c == 0) {
     svo_grafting g;
     g.graft_data_address = 8u * k;
@@ -361,7 +381,7 @@ __global__ __launch_bounds__(kWg) void flag_count_kernel(const uint32_t *flags, 
   }
   const uint32_t i0 = blockIdx.x * kSelChunk + threadIdx.x * kSelPer;
   uint32_t c = 0;
-  for (uint32_t j = 0; j < kSelPer; j++) c += i0 + j < n ? flags[i0 + j] : 0u;
+  for (uint32_t j = 0; j < kSelPer; j++) c += i0 + j < n ? flags[i0 + j] & 1u : 0u;
   uint32_t all;
   wg_scan<kWg>(c, s_waves, &all);
   if (threadIdx.x == 0) counts[blockIdx.x] = all;
@@ -378,7 +398,7 @@ __global__ __launch_bounds__(kWg) void flag_rank_kernel(const uint32_t *flags, u
   const uint32_t i0 = blockIdx.x * kSelChunk + threadIdx.x * kSelPer;
   uint32_t f[kSelPer], c = 0;
   for (uint32_t j = 0; j < kSelPer; j++) {
-    f[j] = i0 + j < n ? flags[i0 + j] : 0u;
+    f[j] = i0 + j < n ? flags[i0 + j] & 1u : 0u;
     c += f[j];
   }
   uint32_t all;
@@ -476,7 +496,9 @@ __device__ __forceinline__ bool has_children_bits(uint32_t chunk) {  // CanHaveC
 
 __device__ __forceinline__ uint32_t spread3_dev(uint32_t v) { return dev::spread3(v); }
 
+template <uint32_t KIND>
 __global__ __launch_bounds__(kWg) void bt_bases_kernel(GeomView g, uint16_t *bases, uint32_t level, uint32_t offset) {
+  g.kind = KIND;
   const uint32_t n = 1u << (3 * level);
   for (uint32_t m = blockIdx.x * kWg + threadIdx.x; m < n; m += gridDim.x * kWg)
     bases[offset + m] = geom_chunk(g, level, compact3(m), compact3(m >> 1), compact3(m >> 2));
@@ -489,37 +511,49 @@ __device__ __forceinline__ bool dense_mixed(const uint16_t *bases, uint32_t B, u
 }
 
 // Dense level L0 = B+2 in x-outer / z-inner order: p = (x << 2s) | (y << s) | z.
-// flag[p] = the block is written and gets children.
+// flag[p] bit 0 = the block is written and gets children; bits 16..31 its chunk, where it is written
+// and the level may have children.
+template <uint32_t KIND>
 __global__ __launch_bounds__(kWg) void bt_dense_flags_kernel(GeomView g, const uint16_t *bases, uint32_t B,
                                                              uint32_t max_depth, uint32_t *flag) {
+  g.kind = KIND;
   const uint32_t L0 = B + 2, n = 1u << (3 * L0), m = (1u << L0) - 1u;
   for (uint32_t p = blockIdx.x * kWg + threadIdx.x; p < n; p += gridDim.x * kWg) {
     const uint32_t x = p >> (2 * L0), y = (p >> L0) & m, z = p & m;
     const uint32_t la = spread3_dev(x) | (spread3_dev(y) << 1) | (spread3_dev(z) << 2);
-    bool f = false;
-    if (L0 < max_depth && dense_mixed(bases, B, la >> 3)) f = has_children_bits(geom_chunk(g, L0, x, y, z));
-    flag[p] = f ? 1u : 0u;
+    uint32_t f = 0;
+    if (L0 < max_depth && dense_mixed(bases, B, la >> 3)) {
+      const uint32_t chunk = geom_chunk(g, L0, x, y, z);
+      f = (chunk << 16) | (has_children_bits(chunk) ? 1u : 0u);
+    }
+    flag[p] = f;
   }
 }
 
 // Level-(B+1) cells in z-outer / x-inner order (PopulateInitialBlocks' loop): mixed[q] with
-// q = (z << 2s) | (y << s) | x; empty[bp] for the free-group FIFO (bp ascending).
+// q = (z << 2s) | (y << s) | x; empty[bp] for the free-group FIFO (bp ascending); *last (cleared
+// before) receives 1 + the largest mixed bp: all eight dense blocks of a mixed cell are written, so
+// the dense level's addresses end at 8 * *last.
 __global__ __launch_bounds__(kWg) void bt_octant_flags_kernel(const uint16_t *bases, uint32_t B, uint32_t *mixed_zyx,
-                                                              uint32_t *empty) {
+                                                              uint32_t *empty, uint32_t *last) {
   const uint32_t S = B + 1, n = 1u << (3 * S), m = (1u << S) - 1u;
+  uint32_t most = 0;
   for (uint32_t q = blockIdx.x * kWg + threadIdx.x; q < n; q += gridDim.x * kWg) {
     const uint32_t z = q >> (2 * S), y = (q >> S) & m, x = q & m;
     const uint32_t bp = spread3_dev(x) | (spread3_dev(y) << 1) | (spread3_dev(z) << 2);
     const bool mx = dense_mixed(bases, B, bp);
     mixed_zyx[q] = mx ? 1u : 0u;
     empty[bp] = mx ? 0u : 1u;
+    if (mx) most = max(most, bp + 1u);
   }
+  for (int off = 32; off > 0; off >>= 1) most = max(most, (uint32_t)__shfl_xor((int)most, off));
+  if ((threadIdx.x & 63u) == 0u && most) atomicMax(last, most);
 }
 
 __global__ __launch_bounds__(kWg) void bt_scatter_index_kernel(const uint32_t *flag, const uint32_t *rank, uint32_t n,
                                                                uint32_t *out) {
   for (uint32_t i = blockIdx.x * kWg + threadIdx.x; i < n; i += gridDim.x * kWg)
-    if (flag[i]) out[rank[i]] = i;
+    if (flag[i] & 1u) out[rank[i]] = i;
 }
 
 // Cells of the internal blocks of the dense level, from their x-outer positions.
@@ -527,30 +561,31 @@ __global__ __launch_bounds__(kWg) void bt_dense_cells_kernel(const uint32_t *fla
                                                              uint3 *cells) {
   const uint32_t n = 1u << (3 * L0), m = (1u << L0) - 1u;
   for (uint32_t p = blockIdx.x * kWg + threadIdx.x; p < n; p += gridDim.x * kWg)
-    if (flag[p]) cells[rank[p]] = make_uint3(p >> (2 * L0), (p >> L0) & m, p & m);
+    if (flag[p] & 1u) cells[rank[p]] = make_uint3(p >> (2 * L0), (p >> L0) & m, p & m);
 }
 
 __device__ __forceinline__ uint3 child_cell(uint3 c, uint32_t i) {
   return make_uint3(2u * c.x + (i & 1u), 2u * c.y + ((i >> 1) & 1u), 2u * c.z + ((i >> 2) & 1u));
 }
 
-// Level L (> L0) nodes: node k is child k & 7 of internal block k >> 3 of level L-1.
+// Level L (L0 < L < the deepest) nodes: node k is child k & 7 of internal block k >> 3 of level L-1.
+// flag[k] bit 0 = it gets children, bits 16..31 its chunk (kept for the write, which would
+// otherwise classify the eight octants again).
+template <uint32_t KIND>
 __global__ __launch_bounds__(kWg) void bt_level_flags_kernel(GeomView g, const uint3 *parent_cells, uint32_t n,
-                                                             uint32_t L, uint32_t max_depth, uint32_t *flag) {
+                                                             uint32_t L, uint32_t *flag) {
+  g.kind = KIND;
   for (uint32_t k = blockIdx.x * kWg + threadIdx.x; k < n; k += gridDim.x * kWg) {
-    bool f = false;
-    if (L < max_depth) {
-      const uint3 c = child_cell(parent_cells[k >> 3], k & 7u);
-      f = has_children_bits(geom_chunk(g, L, c.x, c.y, c.z));
-    }
-    flag[k] = f ? 1u : 0u;
+    const uint3 c = child_cell(parent_cells[k >> 3], k & 7u);
+    const uint32_t chunk = geom_chunk(g, L, c.x, c.y, c.z);
+    flag[k] = (chunk << 16) | (has_children_bits(chunk) ? 1u : 0u);
   }
 }
 
 __global__ __launch_bounds__(kWg) void bt_level_cells_kernel(const uint3 *parent_cells, const uint32_t *flag,
                                                              const uint32_t *rank, uint32_t n, uint3 *cells) {
   for (uint32_t k = blockIdx.x * kWg + threadIdx.x; k < n; k += gridDim.x * kWg)
-    if (flag[k]) cells[rank[k]] = child_cell(parent_cells[k >> 3], k & 7u);
+    if (flag[k] & 1u) cells[rank[k]] = child_cell(parent_cells[k >> 3], k & 7u);
 }
 
 // Bottom-up: allocations (groups) and block writes in the subtree of internal block j.
@@ -562,7 +597,7 @@ __global__ __launch_bounds__(kWg) void bt_sizes_kernel(uint32_t n_int, const uin
     if (cflag) {
       for (uint32_t i = 0; i < 8u; i++) {
         const uint32_t k = 8u * j + i;
-        if (cflag[k]) {
+        if (cflag[k] & 1u) {
           a += calloc[crank[k]];
           w += cwrites[crank[k]];
         }
@@ -584,7 +619,7 @@ __global__ __launch_bounds__(kWg) void bt_ranks_kernel(uint32_t n_int, const uin
     uint32_t r = rank[j] + 1u, w = start[j];
     for (uint32_t i = 0; i < 8u; i++) {
       const uint32_t k = 8u * j + i;
-      if (cflag && cflag[k]) {
+      if (cflag[k] & 1u) {
         const uint32_t c = crank[k];
         child_rank[c] = r;
         child_start[c] = w;
@@ -602,24 +637,22 @@ __device__ __forceinline__ uint32_t fifo_group(const GroupFifo &f, uint32_t r) {
   return r < f.n_empties ? f.empties[r] : f.dense_groups + (r - f.n_empties);
 }
 
-__device__ __forceinline__ void bt_store(const BuildOut &o, uint32_t a, uint4 b, uint32_t post) {
-  o.blocks[a] = b;
-  o.post[a] = post;
-  atomicMax(&o.max[0], (unsigned long long)a);
-}
-
-// The dense level's blocks (written first, in PopulateInitialBlocks' order).
+// The dense level's blocks (written first, in PopulateInitialBlocks' order); with children, `flag`
+// holds the chunks.
+template <uint32_t KIND>
 __global__ __launch_bounds__(kWg) void bt_write_dense_kernel(GeomView g, const uint16_t *bases, uint32_t B,
                                                              const uint32_t *flag, const uint32_t *irank,
                                                              const uint32_t *rank, const uint32_t *mixed_rank,
-                                                             GroupFifo fifo, BuildOut o) {
+                                                             uint32_t children, GroupFifo fifo, BuildOut o) {
+  g.kind = KIND;
   const uint32_t L0 = B + 2, n = 1u << (3 * L0), m = (1u << L0) - 1u, S = B + 1;
   for (uint32_t p = blockIdx.x * kWg + threadIdx.x; p < n; p += gridDim.x * kWg) {
     const uint32_t x = p >> (2 * L0), y = (p >> L0) & m, z = p & m;
     const uint32_t la = spread3_dev(x) | (spread3_dev(y) << 1) | (spread3_dev(z) << 2);
     if (!dense_mixed(bases, B, la >> 3)) continue;
-    uint4 b = geom_block(g, L0, x, y, z);
-    if (flag[p]) {
+    const uint32_t f = flag[p];
+    uint4 b = geom_block(g, L0, x, y, z, children != 0u, f >> 16);
+    if (f & 1u) {
       const uint32_t r = rank[irank[p]];
       if (r < fifo.capacity) {
         const uint32_t g = fifo_group(fifo, r);
@@ -628,24 +661,31 @@ __global__ __launch_bounds__(kWg) void bt_write_dense_kernel(GeomView g, const u
       }
     }
     const uint32_t q = ((z >> 1) << (2 * S)) | ((y >> 1) << S) | (x >> 1);  // its level-(B+1) cell, z-outer
-    bt_store(o, la, b, 8u * mixed_rank[q] + (la & 7u));
-    atomicMax(&o.max[1], (unsigned long long)la);
+    o.blocks[la] = b;
+    o.post[la] = 8u * mixed_rank[q] + (la & 7u);
   }
 }
 
-// Level L (> L0) nodes whose parent got its group.
+// Level L (> L0) nodes whose parent got its group.  The deepest level has no flags, ranks or write
+// positions of its own: its blocks are childless, and block k's position is its parent's first one
+// plus its octant.  (Every thread used to raise one address to the largest block written; the
+// atomics took 6 of the 7.2 ms of the 40 M blocks of a depth-12 heightfield's deepest level.  The
+// largest address follows from the FIFO entries taken, on the host.)
+template <uint32_t KIND>
 __global__ __launch_bounds__(kWg) void bt_write_level_kernel(GeomView g, const uint3 *parent_cells,
-                                                             const uint32_t *parent_rank, uint32_t n, uint32_t L,
-                                                             const uint32_t *flag, const uint32_t *irank,
-                                                             const uint32_t *rank, const uint32_t *post,
-                                                             GroupFifo fifo, BuildOut o) {
+                                                             const uint32_t *parent_rank, const uint32_t *parent_start,
+                                                             uint32_t n, uint32_t L, const uint32_t *flag,
+                                                             const uint32_t *irank, const uint32_t *rank,
+                                                             const uint32_t *post, GroupFifo fifo, BuildOut o) {
+  g.kind = KIND;
   for (uint32_t k = blockIdx.x * kWg + threadIdx.x; k < n; k += gridDim.x * kWg) {
     const uint32_t pr = parent_rank[k >> 3];
     if (pr >= fifo.capacity) continue;  // the FIFO ran out before the parent's group
     const uint32_t a = (fifo_group(fifo, pr) << 3) + (k & 7u);
     const uint3 c = child_cell(parent_cells[k >> 3], k & 7u);
-    uint4 b = geom_block(g, L, c.x, c.y, c.z);
-    if (flag && flag[k]) {
+    const uint32_t f = flag ? flag[k] : 0u;
+    uint4 b = geom_block(g, L, c.x, c.y, c.z, flag != nullptr, f >> 16);
+    if (f & 1u) {
       const uint32_t r = rank[irank[k]];
       if (r < fifo.capacity) {
         const uint32_t g = fifo_group(fifo, r);
@@ -653,7 +693,8 @@ __global__ __launch_bounds__(kWg) void bt_write_level_kernel(GeomView g, const u
         o.group_parent[g] = a;
       }
     }
-    bt_store(o, a, b, post[k]);
+    o.blocks[a] = b;
+    o.post[a] = flag ? post[k] : parent_start[k >> 3] + (k & 7u);
   }
 }
 
@@ -778,24 +819,41 @@ int launch_compact_moves(const PoolView &p, const uint32_t *from, const uint32_t
 
 // ---- device TreeBuilder ----
 
+// A kernel for each kind of geometry: the noise's registers do not limit the other kinds' occupancy.
+#define BT_LAUNCH(kernel, ...)                                                                                  \
+  switch (g.kind) {                                                                                             \
+    case SVO_GEOMETRY_FBM_HEIGHTFIELD:                                                                          \
+      hipLaunchKernelGGL((kernel<SVO_GEOMETRY_FBM_HEIGHTFIELD>), __VA_ARGS__);                                   \
+      break;                                                                                                    \
+    case SVO_GEOMETRY_SPHERES:                                                                                  \
+      hipLaunchKernelGGL((kernel<SVO_GEOMETRY_SPHERES>), __VA_ARGS__);                                           \
+      break;                                                                                                    \
+    case SVO_GEOMETRY_CUBES:                                                                                    \
+      hipLaunchKernelGGL((kernel<SVO_GEOMETRY_CUBES>), __VA_ARGS__);                                             \
+      break;                                                                                                    \
+    default:                                                                                                    \
+      hipLaunchKernelGGL((kernel<SVO_GEOMETRY_SPHERE_NOISE>), __VA_ARGS__);                                      \
+  }
+
 int launch_bt_bases(const GeomView &g, uint16_t *bases, uint32_t B, hipStream_t s) {
   for (uint32_t d = 1; d <= B; d++) {
     const uint32_t offset = ((1u << (3u * d)) - 1u) / 7u - 1u;  // powSum(d-1)
-    hipLaunchKernelGGL(bt_bases_kernel, dim3(grid_for(1ull << (3 * d))), dim3(kWg), 0, s, g, bases, d, offset);
+    BT_LAUNCH(bt_bases_kernel, dim3(grid_for(1ull << (3 * d))), dim3(kWg), 0, s, g, bases, d, offset);
     if (rc_of()) return -1;
   }
   return 0;
 }
 
-int launch_bt_octant_flags(const uint16_t *bases, uint32_t B, uint32_t *mixed_zyx, uint32_t *empty, hipStream_t s) {
+int launch_bt_octant_flags(const uint16_t *bases, uint32_t B, uint32_t *mixed_zyx, uint32_t *empty, uint32_t *last,
+                           hipStream_t s) {
   hipLaunchKernelGGL(bt_octant_flags_kernel, dim3(grid_for(1ull << (3 * (B + 1)))), dim3(kWg), 0, s, bases, B,
-                     mixed_zyx, empty);
+                     mixed_zyx, empty, last);
   return rc_of();
 }
 
 int launch_bt_dense_flags(const GeomView &g, const uint16_t *bases, uint32_t B, uint32_t max_depth, uint32_t *flag,
                           hipStream_t s) {
-  hipLaunchKernelGGL(bt_dense_flags_kernel, dim3(grid_for(1ull << (3 * (B + 2)))), dim3(kWg), 0, s, g, bases, B,
+  BT_LAUNCH(bt_dense_flags_kernel, dim3(grid_for(1ull << (3 * (B + 2)))), dim3(kWg), 0, s, g, bases, B,
                      max_depth, flag);
   return rc_of();
 }
@@ -811,10 +869,10 @@ int launch_bt_dense_cells(const uint32_t *flag, const uint32_t *rank, uint32_t L
   return rc_of();
 }
 
-int launch_bt_level_flags(const GeomView &g, const uint3 *parent_cells, uint32_t n, uint32_t L, uint32_t max_depth,
-                          uint32_t *flag, hipStream_t s) {
+int launch_bt_level_flags(const GeomView &g, const uint3 *parent_cells, uint32_t n, uint32_t L, uint32_t *flag,
+                          hipStream_t s) {
   if (!n) return 0;
-  hipLaunchKernelGGL(bt_level_flags_kernel, dim3(grid_for(n)), dim3(kWg), 0, s, g, parent_cells, n, L, max_depth, flag);
+  BT_LAUNCH(bt_level_flags_kernel, dim3(grid_for(n)), dim3(kWg), 0, s, g, parent_cells, n, L, flag);
   return rc_of();
 }
 
@@ -843,19 +901,20 @@ int launch_bt_ranks(uint32_t n_int, const uint32_t *rank, const uint32_t *start,
 }
 
 int launch_bt_write_dense(const GeomView &g, const uint16_t *bases, uint32_t B, const uint32_t *flag,
-                          const uint32_t *irank, const uint32_t *rank, const uint32_t *mixed_rank,
+                          const uint32_t *irank, const uint32_t *rank, const uint32_t *mixed_rank, bool children,
                           const GroupFifo &fifo, const BuildOut &o, hipStream_t s) {
-  hipLaunchKernelGGL(bt_write_dense_kernel, dim3(grid_for(1ull << (3 * (B + 2)))), dim3(kWg), 0, s, g, bases, B, flag,
-                     irank, rank, mixed_rank, fifo, o);
+  BT_LAUNCH(bt_write_dense_kernel, dim3(grid_for(1ull << (3 * (B + 2)))), dim3(kWg), 0, s, g, bases, B, flag,
+                     irank, rank, mixed_rank, children ? 1u : 0u, fifo, o);
   return rc_of();
 }
 
-int launch_bt_write_level(const GeomView &g, const uint3 *parent_cells, const uint32_t *parent_rank, uint32_t n,
-                          uint32_t L, const uint32_t *flag, const uint32_t *irank, const uint32_t *rank,
-                          const uint32_t *post, const GroupFifo &fifo, const BuildOut &o, hipStream_t s) {
+int launch_bt_write_level(const GeomView &g, const uint3 *parent_cells, const uint32_t *parent_rank,
+                          const uint32_t *parent_start, uint32_t n, uint32_t L, const uint32_t *flag,
+                          const uint32_t *irank, const uint32_t *rank, const uint32_t *post, const GroupFifo &fifo,
+                          const BuildOut &o, hipStream_t s) {
   if (!n) return 0;
-  hipLaunchKernelGGL(bt_write_level_kernel, dim3(grid_for(n)), dim3(kWg), 0, s, g, parent_cells, parent_rank, n, L,
-                     flag, irank, rank, post, fifo, o);
+  BT_LAUNCH(bt_write_level_kernel, dim3(grid_for(n)), dim3(kWg), 0, s, g, parent_cells, parent_rank,
+                     parent_start, n, L, flag, irank, rank, post, fifo, o);
   return rc_of();
 }
 

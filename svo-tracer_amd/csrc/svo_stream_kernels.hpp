@@ -88,36 +88,41 @@ struct GroupFifo {
 // Outputs of the write kernels.
 struct BuildOut {
   uint4 *blocks;
-  uint32_t *post;           // per block address: position in TreeBuilder's write sequence (phase-local)
-  uint32_t *group_parent;   // per group: the block whose children it holds
-  unsigned long long *max;  // [0] largest address written, [1] largest dense-level address written
+  uint32_t *post;          // per block address: position in TreeBuilder's write sequence (phase-local)
+  uint32_t *group_parent;  // per group: the block whose children it holds
 };
 int launch_bt_bases(const GeomView &g, uint16_t *bases, uint32_t B, hipStream_t s);
-// Level-(B+1) cells: mixed_zyx in z-outer / x-inner order, empty by Morton index.
-int launch_bt_octant_flags(const uint16_t *bases, uint32_t B, uint32_t *mixed_zyx, uint32_t *empty, hipStream_t s);
-// Dense level in x-outer / z-inner order: the written blocks that get children.
+// Level-(B+1) cells: mixed_zyx in z-outer / x-inner order, empty by Morton index; *last (cleared
+// before) receives 1 + the largest mixed Morton index.
+int launch_bt_octant_flags(const uint16_t *bases, uint32_t B, uint32_t *mixed_zyx, uint32_t *empty, uint32_t *last,
+                           hipStream_t s);
+// Dense level in x-outer / z-inner order: the written blocks that get children (bit 0), and their
+// chunks (bits 16..31, when B+2 < max_depth).
 int launch_bt_dense_flags(const GeomView &g, const uint16_t *bases, uint32_t B, uint32_t max_depth, uint32_t *flag,
                           hipStream_t s);
 int launch_bt_scatter_index(const uint32_t *flag, const uint32_t *rank, uint32_t n, uint32_t *out, hipStream_t s);
 int launch_bt_dense_cells(const uint32_t *flag, const uint32_t *rank, uint32_t L0, uint3 *cells, hipStream_t s);
-// Level L's nodes (child k & 7 of internal block k >> 3 of level L-1): those that get children.
-int launch_bt_level_flags(const GeomView &g, const uint3 *parent_cells, uint32_t n, uint32_t L, uint32_t max_depth,
-                          uint32_t *flag, hipStream_t s);
+// Level L's nodes (child k & 7 of internal block k >> 3 of level L-1): those that get children
+// (bit 0), and their chunks (bits 16..31).
+int launch_bt_level_flags(const GeomView &g, const uint3 *parent_cells, uint32_t n, uint32_t L, uint32_t *flag,
+                          hipStream_t s);
 int launch_bt_level_cells(const uint3 *parent_cells, const uint32_t *flag, const uint32_t *rank, uint32_t n,
                           uint3 *cells, hipStream_t s);
 // Subtree allocations and writes of each internal block (cflag null: no internal children).
 int launch_bt_sizes(uint32_t n_int, const uint32_t *cflag, const uint32_t *crank, const uint32_t *calloc,
                     const uint32_t *cwrites, uint32_t *alloc, uint32_t *writes, hipStream_t s);
-// Ranks and write positions of the next level from this level's.
+// Ranks and write positions of the next level (one that has flags) from this level's.
 int launch_bt_ranks(uint32_t n_int, const uint32_t *rank, const uint32_t *start, const uint32_t *cflag,
                     const uint32_t *crank, const uint32_t *calloc, const uint32_t *cwrites, uint32_t *child_rank,
                     uint32_t *child_start, uint32_t *child_post, hipStream_t s);
 int launch_bt_write_dense(const GeomView &g, const uint16_t *bases, uint32_t B, const uint32_t *flag,
-                          const uint32_t *irank, const uint32_t *rank, const uint32_t *mixed_rank,
+                          const uint32_t *irank, const uint32_t *rank, const uint32_t *mixed_rank, bool children,
                           const GroupFifo &fifo, const BuildOut &o, hipStream_t s);
-int launch_bt_write_level(const GeomView &g, const uint3 *parent_cells, const uint32_t *parent_rank, uint32_t n,
-                          uint32_t L, const uint32_t *flag, const uint32_t *irank, const uint32_t *rank,
-                          const uint32_t *post, const GroupFifo &fifo, const BuildOut &o, hipStream_t s);
+// flag null: the deepest level, without flags, ranks or write positions of its own.
+int launch_bt_write_level(const GeomView &g, const uint3 *parent_cells, const uint32_t *parent_rank,
+                          const uint32_t *parent_start, uint32_t n, uint32_t L, const uint32_t *flag,
+                          const uint32_t *irank, const uint32_t *rank, const uint32_t *post, const GroupFifo &fifo,
+                          const BuildOut &o, hipStream_t s);
 int launch_bt_usages(const uint32_t *group_parent, uint32_t n_groups, uint32_t dense_groups, uint32_t tick,
                      svo_usage *u, hipStream_t s);
 
