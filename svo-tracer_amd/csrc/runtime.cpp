@@ -39,7 +39,7 @@ int hip_fail(hipError_t e, const char *what) {
 
 int new_buffer(size_t bytes, std::shared_ptr<DeviceBuffer> *out) {
   auto b = std::make_shared<DeviceBuffer>();
-  b->bytes = bytes;
+  b->bytes = b->capacity = bytes;
   if (bytes) {
     hipError_t e = hipMalloc(&b->ptr, bytes);
     if (e != hipSuccess) return hip_fail(e, "hipMalloc");

@@ -499,29 +499,71 @@ struct BuildLevel {
 };
 
 // The build's temporaries are carved from a few slabs, each four times the last one's size (up to
-// 512 MiB) or what the piece needs, all released at the end: some fifty allocations and as many
-// frees of a depth-12 build (70 and 180 us each) took as long as its kernels.
+// 256 MiB) or what the piece needs.  Some fifty allocations and as many frees of a depth-12 build
+// (70 and 180 us each, and many milliseconds each when the driver has to give memory back first)
+// took longer than its kernels, so a build that succeeds leaves up to kKeptBuildBytes of its slabs
+// to the context for the next one.
+constexpr size_t kKeptBuildBytes = (size_t)512 << 20;
+
 struct Builder {
   Context *ctx;
   hipStream_t s;
-  std::vector<std::shared_ptr<DeviceBuffer>> slabs;
+  std::vector<std::shared_ptr<DeviceBuffer>> slabs, kept;
   size_t used = 0, next = (size_t)32 << 20;
+
+  explicit Builder(Context *c) : ctx(c), s(c->stream), kept(std::move(c->build_slabs)) { c->build_slabs.clear(); }
 
   int buf(size_t bytes, Piece *out) {
     bytes = (std::max<size_t>(bytes, 4) + 255) & ~(size_t)255;
     if (slabs.empty() || bytes > slabs.back()->bytes - used) {
       std::shared_ptr<DeviceBuffer> slab;
-      int rc = new_buffer(std::max(bytes, next), &slab);
-      if (rc && bytes < next) rc = new_buffer(bytes, &slab);
-      if (rc) return rc;
+      // the first kept slab that holds the piece, or a new one
+      for (auto k = kept.begin(); k != kept.end() && !slab; ++k)
+        if ((*k)->bytes >= bytes) {
+          slab = *k;
+          kept.erase(k);
+          break;
+        }
+      if (!slab) {
+        int rc = new_buffer(std::max(bytes, next), &slab);
+        if (rc) {
+          kept.clear();
+          rc = new_buffer(bytes, &slab);
+        }
+        if (rc) return rc;
+      }
       slabs.push_back(slab);
       used = 0;
-      next = std::min(4 * next, (size_t)512 << 20);
+      next = std::min(4 * next, (size_t)256 << 20);
     }
     out->ptr = (char *)slabs.back()->ptr + used;
     out->bytes = bytes;
     used += bytes;
     return SVO_OK;
+  }
+  // Leaves the slabs to the context (the stream orders the next build's use of them after this
+  // one's).
+  void keep() {
+    size_t total = 0;
+    for (auto *from : {&slabs, &kept})
+      for (auto &b : *from)
+        if (total + b->bytes <= kKeptBuildBytes) {
+          total += b->bytes;
+          ctx->build_slabs.push_back(b);
+        }
+  }
+  // A named buffer of `bytes`: the context's own when nothing else holds it and it fits (and is no
+  // more than twice as large), a new one otherwise.  *in_place: the caller's other streams may
+  // still read it.
+  int named(int name, size_t bytes, std::shared_ptr<DeviceBuffer> *out, bool *in_place) {
+    auto it = ctx->buffers.find(name);
+    if (it != ctx->buffers.end() && it->second && it->second.use_count() == 1 && bytes &&
+        it->second->capacity >= bytes && it->second->capacity <= 2 * bytes) {
+      *out = it->second;
+      *in_place = true;
+      return SVO_OK;
+    }
+    return new_buffer(bytes, out);
   }
   template <class T>
   T *ptr(const Piece &b) {
@@ -561,7 +603,7 @@ namespace {
 
 int build_tree_device(Context *ctx, const GeomView &g, uint32_t base_depth, uint32_t max_depth, uint32_t max_size,
                       int with_usages, uint16_t usage_tick, svo_tree **out, uint32_t *block_count) {
-  Builder bd{ctx, ctx->stream, {}};
+  Builder bd(ctx);
   const uint32_t B = base_depth, L0 = B + 2;
   const uint32_t dense_groups = 1u << (3 * (B + 1)), n0 = 1u << (3 * L0);
   // FIFO length, as TreeBuilder.BuildTree sizes it (maxSize at least the dense level)
@@ -690,11 +732,17 @@ int build_tree_device(Context *ctx, const GeomView &g, uint32_t base_depth, uint
   const uint64_t groups64 = dense_groups + (taken > n_empties ? taken - n_empties : 0);
   if (groups64 * 8 > 0xffffffffull) return fail(SVO_ERR_CAPACITY, "svo_terrain_build_tree: more than 2^32 blocks");
   const uint32_t n_groups = (uint32_t)groups64;
-  std::shared_ptr<DeviceBuffer> blocks;
+  // Everything that can be refused has been.  A tree of about the last one's size is written over
+  // it, after whatever still reads that (as freeing it would wait).
+  std::shared_ptr<DeviceBuffer> blocks, usages;
   Piece post, gparent;
-  if ((rc = new_buffer((size_t)n_groups * 128, &blocks)) || (rc = bd.buf((size_t)n_groups * 32, &post)) ||
-      (rc = bd.buf((size_t)n_groups * 4, &gparent)))
+  bool in_place = false;
+  if ((rc = bd.named(SVO_BUF_BLOCKS, (size_t)n_groups * 128, &blocks, &in_place)) ||
+      (with_usages && (rc = bd.named(SVO_BUF_USAGES, (size_t)n_groups * sizeof(svo_usage), &usages, &in_place))) ||
+      (rc = bd.buf((size_t)n_groups * 32, &post)) || (rc = bd.buf((size_t)n_groups * 4, &gparent)))
     return rc;
+  if (in_place && hipDeviceSynchronize() != hipSuccess)
+    return hip_fail(hipGetLastError(), "svo_terrain_build_tree: sync");
   // only the dense groups can stay unwritten: every other group in use is a FIFO entry that was
   // taken, with a parent and eight blocks
   if ((rc = bd.fill(blocks->ptr, 0, (size_t)dense_groups * 128)) ||
@@ -776,12 +824,12 @@ int build_tree_device(Context *ctx, const GeomView &g, uint32_t base_depth, uint
     return rc;
   bases_out->flags = SVO_BUFFER_READ_ONLY;
   blocks->flags = SVO_BUFFER_READ_ONLY;
-  std::shared_ptr<DeviceBuffer> cu;
   if (with_usages) {
-    if ((rc = new_buffer((size_t)out_groups * sizeof(svo_usage), &cu))) return rc;
-    cu->flags = SVO_BUFFER_READ_WRITE;
+    usages->bytes = (size_t)out_groups * sizeof(svo_usage);
+    usages->flags = SVO_BUFFER_READ_WRITE;
+    if (!out_groups && (rc = new_buffer(0, &usages))) return rc;
     if ((rc = bd.launched(launch_bt_usages(bd.ptr<uint32_t>(gparent), out_groups, dense_groups, usage_tick,
-                                           (svo_usage *)cu->ptr, bd.s),
+                                           (svo_usage *)usages->ptr, bd.s),
                           "usages")))
       return rc;
   }
@@ -802,7 +850,8 @@ int build_tree_device(Context *ctx, const GeomView &g, uint32_t base_depth, uint
   if (e != hipSuccess) return hip_fail(e, "svo_terrain_build_tree");
   ctx->buffers[SVO_BUF_BASES] = bases_out;
   ctx->buffers[SVO_BUF_BLOCKS] = blocks;
-  if (cu) ctx->buffers[SVO_BUF_USAGES] = cu;
+  if (usages) ctx->buffers[SVO_BUF_USAGES] = usages;
+  bd.keep();
   ctx->tree_max_depth = max_depth;
   return SVO_OK;
 }

@@ -17,6 +17,7 @@ namespace svo {
 struct DeviceBuffer {
   void *ptr = nullptr;
   size_t bytes = 0;
+  size_t capacity = 0;  // bytes allocated (at least `bytes`)
   uint32_t flags = 0;
   ~DeviceBuffer();
 };
@@ -158,6 +159,8 @@ struct Context {
   } kept;
   // span sums of the multi-work-group scans (tree management, streaming, device builds)
   std::shared_ptr<DeviceBuffer> scan_sums;
+  // temporaries of the last device build, kept for the next one (at most kKeptBuildBytes)
+  std::vector<std::shared_ptr<DeviceBuffer>> build_slabs;
   uint32_t *id_host = nullptr;  // pinned word for the queue-counter read-backs (svo_reset_id)
   // batched cameras: concatenated camera tables (cache key), camera records
   std::shared_ptr<DeviceBuffer> scratch_batch_lut;

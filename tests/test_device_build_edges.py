@@ -52,3 +52,33 @@ def test_equals_host_build(svo, gpu, name, below):
     assert np.array_equal(gpu.ReadBuffer(B.Blocks, np.uint8), ref.blocks.view(np.uint8))
     assert np.array_equal(gpu.ReadBuffer(B.Usages, svo.USAGE_DTYPE), ref.initial_usages(3))
 
+
+
+def test_rebuilds_in_place(svo, gpu):
+    """Builds over the last build's buffers (about the same size, nothing else holding them), over
+    buffers that a kernel argument still holds (which are left alone), and of other sizes."""
+    B, K = svo.BufferName, svo.KernelName
+    big = 0xFFFFFFFF // 8
+
+    def build(spec, depth, tick):
+        ref = svo.build_tree(spec.geometry, spec.base_depth, depth, big)
+        gpu.BuildTreeDevice(spec.geometry, spec.base_depth, depth, big, with_usages=True, usage_tick=tick)
+        assert np.array_equal(gpu.ReadBuffer(B.Blocks, np.uint8), ref.blocks.view(np.uint8))
+        assert np.array_equal(gpu.ReadBuffer(B.Bases, np.uint16), ref.bases)
+        assert np.array_equal(gpu.ReadBuffer(B.Usages, svo.USAGE_DTYPE), ref.initial_usages(tick))
+
+    hills, steep = heightfield(svo), heightfield(svo, seed=8, z_min=0.3, z_max=0.5)
+    build(hills, 8, 1)
+    first = gpu.DevicePointer(B.Blocks)
+    build(hills, 8, 2)
+    assert gpu.DevicePointer(B.Blocks) == first
+    build(steep, 8, 3)
+    gpu.SetArg(K.ResolveRemainders, "Blocks", B.Blocks)  # the argument holds this build's blocks
+    held = gpu.DevicePointer(B.Blocks)
+    build(hills, 8, 4)
+    assert gpu.DevicePointer(B.Blocks) != held
+    gpu.InitBuffer(B.PruningBlockData, np.zeros(1, svo.BLOCK_DTYPE))
+    gpu.SetArg(K.ResolveRemainders, "Blocks", B.PruningBlockData)
+    build(hills, 6, 5)
+    build(steep, 9, 6)
+    build(noise(svo), 5, 7)
