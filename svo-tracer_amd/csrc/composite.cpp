@@ -91,7 +91,7 @@ extern "C" int svo_composite(svo_context *ctx, const svo_trace_input *views, con
   int per_cu = 0;
   if (composite_occupancy(plan.shape.lds_bytes, &per_cu) != 0 || per_cu <= 0)
     return fail(SVO_ERR_HIP, "svo_composite: occupancy query failed");
-  plan.shape.grid = std::max(8, (per_cu * std::max(1, ctx->cu_count) / 8) * 8);
+  plan.shape.grid = std::min(plan.shape.max_grid, std::max(8, (per_cu * std::max(1, ctx->cu_count) / 8) * 8));
 
   const uint32_t n_inline = n_views <= kInlineCams ? n_views : 0u;
   if (!n_inline) {

@@ -74,6 +74,7 @@ struct FrameParams {
   uint32_t stack_levels;
   uint32_t ticked_slots;  // slots of the LDS table of ticked usage groups (0: no table)
   uint32_t refill;
+  uint32_t lanes;  // lanes of a wave that take cones, a power of two (64: all)
   uint32_t chunk;  // work items a wave claims per atomic (multiple of 64)
   // tile schedule (may be null): position k of a band's work range holds tile order[k]; a
   // wave stores the loop iterations it spent on a tile in tile_cost[tile]
@@ -85,6 +86,7 @@ struct LaunchShape {
   int workgroup;
   int waves;  // register budget: waves per SIMD the kernel is compiled for (6)
   int grid;
+  int max_grid;  // work-groups that can find work
   size_t lds_bytes;
   uint32_t ticked_slots;  // the ticked-group table within lds_bytes
 };

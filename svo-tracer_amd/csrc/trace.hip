@@ -62,13 +62,17 @@ __global__ void __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(WAVES >
 trace_frame_kernel(const FrameParams p) {
   extern __shared__ uint32_t smem[];
   uint16_t *s_bases = reinterpret_cast<uint16_t *>(smem);
-  const uint32_t bases_words = p.bases_in_lds ? (p.n_bases + 1u) / 2u : 0u;
+  const uint32_t bases_words = p.bases_in_lds ? p.n_bases / 2u : 0u;
   uint32_t *s_cam = smem + bases_words;
   const uint32_t cam_words = p.n_cams * kCamWords;
   uint32_t *s_ticked = s_cam + cam_words;
   uint32_t *s_stack = s_ticked + p.ticked_slots;
   if (p.bases_in_lds) {
-    for (uint32_t i = threadIdx.x; i < p.n_bases; i += WG) s_bases[i] = p.bases[i];
+    // 16 bytes a load (Bases holds a multiple of 8 chunks and starts an allocation): chunk by chunk
+    // the 18 dependent rounds of a BaseDepth-4 tree delayed every work-group's first cone
+    const uint4 *src = reinterpret_cast<const uint4 *>(p.bases);
+    uint4 *dst = reinterpret_cast<uint4 *>(s_bases);
+    for (uint32_t i = threadIdx.x; i < p.n_bases / 8u; i += WG) dst[i] = src[i];
   }
   {
     const uint32_t *src = reinterpret_cast<const uint32_t *>(p.cams);
@@ -540,10 +544,10 @@ trace_frame_kernel(const FrameParams p) {
 
   for (;;) {
     // ---- refill idle lanes with new cones (wave-uniform control flow) ----
-    const uint64_t idle = __ballot(!active);
+    const uint64_t idle = __ballot(!active && lane < p.lanes);
     const uint32_t n_idle = (uint32_t)__popcll(idle);
     bool fast_cone = false;  // the lane's cone may take fast steps
-    if (fetching && (n_idle >= p.refill || n_idle == 64u)) {
+    if (fetching && (n_idle >= p.refill || n_idle == p.lanes)) {
       flush();
       record_cost();
       // claim a slice of `chunk` work items with one atomic when the wave's slice is used up
@@ -568,7 +572,7 @@ trace_frame_kernel(const FrameParams p) {
         const uint32_t take = min(n_idle, cur_end - cur);
         cur_tile = p.order ? p.order[cur_t0 + (cur >> 6)] : cur_t0 + (cur >> 6);
         cur += take;
-        if (!active && k < cur_end) {
+        if (!active && lane < p.lanes && k < cur_end) {
           uint32_t tile = cur_t0 + (k >> 6);
           if (p.order) tile = p.order[tile];
           const uint32_t l = k & 63u;
@@ -642,7 +646,7 @@ trace_frame_kernel(const FrameParams p) {
     }
     // All lanes were refilled together from one tile (its cones share a camera): fast steps
     // while every one of them is an ordinary cone.
-    if (p.refill >= 64u && n_idle == 64u && __ballot(active && !fast_cone) == 0ull) {
+    if (p.refill >= 64u && n_idle == p.lanes && __ballot(active && !fast_cone) == 0ull) {
       const int lead = __ffsll((unsigned long long)__ballot(active)) - 1;
       cam = (uint32_t)__builtin_amdgcn_readlane((int)cam, lead);
       fov32 = camf(cam, 12) * 2.3283064365386963e-10f;
@@ -976,15 +980,32 @@ __device__ __forceinline__ uint32_t rank_below(uint64_t m) {
 // in 16 rounds of 64 consecutive ids, one per lane: each round's entries of a queue go to
 // consecutive positions (ranks from ballots), so the record reads and the queue writes are
 // coalesced.  Positions continue the chunk offsets of the scan in ascending cone id.
-// fused (at most kFusedChunks chunks): `offsets` holds the chunks' own counts, each work-group
+// kFused (at most kFusedChunks chunks): `offsets` holds the chunks' own counts, each work-group
 // sums those before it, and the last one writes the queue counters and the request total.
-constexpr uint32_t kFusedChunks = 1024;
+// kDirect (at most kDirectChunks chunks): there are no counts; each work-group counts the status
+// bytes before its own.  One launch fewer: about 9 us of a small frame's 80 to 150, against at most
+// 15 x 4096 bytes read again by the last work-group.
+constexpr uint32_t kFusedChunks = 1024, kDirectChunks = 16;
+enum : uint32_t { kScanned = 0, kFused = 1, kDirect = 2 };
 __global__ void __launch_bounds__(kCompactThreads) status_scatter_kernel(
     const uint8_t *status, uint32_t n, const uint32_t *offsets, uint32_t *bg_queue, uint32_t *mat_queue,
     const svo_child_request *req_sparse, svo_child_request *requests, uint32_t *req_cones, uint32_t req_capacity,
-    uint32_t fused, uint32_t *bg_count, uint32_t *mat_count, uint32_t *req_count, unsigned long long *totals) {
+    uint32_t mode, uint32_t *bg_count, uint32_t *mat_count, uint32_t *req_count, unsigned long long *totals) {
   uint32_t pre[3];
-  if (fused) {
+  if (mode == kDirect) {
+    uint32_t v[3] = {0u, 0u, 0u};
+    // (all of these bytes lie before this chunk, so none is past the end)
+    for (uint32_t i = threadIdx.x * 16u; i < blockIdx.x * kCompactChunk; i += kCompactThreads * 16u) {
+      uint8_t s[16];
+      load_status16(status, n, i, s);
+#pragma unroll
+      for (int k = 0; k < 16; k++) {
+        const uint32_t c = categories(s[k]);
+        for (int q = 0; q < 3; q++) v[q] += (c >> q) & 1u;
+      }
+    }
+    block_scan3(v, pre);
+  } else if (mode == kFused) {
     uint32_t v[3] = {0u, 0u, 0u};
     for (uint32_t c = threadIdx.x; c < blockIdx.x; c += kCompactThreads)
       for (int q = 0; q < 3; q++) v[q] += offsets[4u * c + q];
@@ -1015,7 +1036,7 @@ __global__ void __launch_bounds__(kCompactThreads) status_scatter_kernel(
     pos[q] = pre[q];
     for (uint32_t w = 0; w < wave; w++) pos[q] += s_tot[q][w];
   }
-  if (fused && blockIdx.x == gridDim.x - 1u && threadIdx.x == 0) {
+  if (mode != kScanned && blockIdx.x == gridDim.x - 1u && threadIdx.x == 0) {
     uint32_t all[3] = {pre[0], pre[1], pre[2]};
     for (uint32_t q = 0; q < 3; q++)
       for (uint32_t w = 0; w < kCompactThreads / 64; w++) all[q] += s_tot[q][w];
@@ -1164,17 +1185,18 @@ uint32_t compaction_chunks(uint32_t n) { return (n + kCompactChunk - 1u) / kComp
 int launch_compaction(const CompactParams &c, hipStream_t stream) {
   const uint32_t chunks = compaction_chunks(c.n);
   if (chunks == 0) return 0;
-  hipLaunchKernelGGL(status_count_kernel, dim3(chunks), dim3(kCompactThreads), 0, stream, c.status, c.n, c.counts);
+  if (chunks > kDirectChunks)
+    hipLaunchKernelGGL(status_count_kernel, dim3(chunks), dim3(kCompactThreads), 0, stream, c.status, c.n, c.counts);
   if (chunks <= kFusedChunks) {
     hipLaunchKernelGGL(status_scatter_kernel, dim3(chunks), dim3(kCompactThreads), 0, stream, c.status, c.n, c.counts,
-                       c.bg_queue, c.mat_queue, c.req_sparse, c.requests, c.req_cones, c.req_capacity, 1u, c.bg_count,
-                       c.mat_count, c.req_count, c.totals);
+                       c.bg_queue, c.mat_queue, c.req_sparse, c.requests, c.req_cones, c.req_capacity,
+                       chunks > kDirectChunks ? kFused : kDirect, c.bg_count, c.mat_count, c.req_count, c.totals);
     return hipGetLastError() == hipSuccess ? 0 : -1;
   }
   hipLaunchKernelGGL(status_scan_kernel, dim3(1), dim3(kCompactThreads), 0, stream, c.counts, chunks, c.bg_count,
                      c.mat_count, c.req_count, c.totals);
   hipLaunchKernelGGL(status_scatter_kernel, dim3(chunks), dim3(kCompactThreads), 0, stream, c.status, c.n, c.counts,
-                     c.bg_queue, c.mat_queue, c.req_sparse, c.requests, c.req_cones, c.req_capacity, 0u, c.bg_count,
+                     c.bg_queue, c.mat_queue, c.req_sparse, c.requests, c.req_cones, c.req_capacity, kScanned, c.bg_count,
                      c.mat_count, c.req_count, c.totals);
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
