@@ -161,7 +161,8 @@ struct Context {
   std::shared_ptr<DeviceBuffer> scan_sums;
   // temporaries of the last device build, kept for the next one (at most kKeptBuildBytes)
   std::vector<std::shared_ptr<DeviceBuffer>> build_slabs;
-  uint32_t *id_host = nullptr;  // pinned word for the queue-counter read-backs (svo_reset_id)
+  unsigned long long *id_host = nullptr;  // pinned word of the queue-counter read-backs (svo_reset_id)
+  uint32_t id_tag = 0;                    // the last read-back's number
   // batched cameras: concatenated camera tables (cache key), camera records
   std::shared_ptr<DeviceBuffer> scratch_batch_lut;
   std::vector<float> batch_lut_key;

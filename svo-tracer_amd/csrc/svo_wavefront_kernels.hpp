@@ -38,14 +38,11 @@ struct InitParams {
   uint32_t W, H, gsx, gsy;
   uint8_t *colour_r, *colour_g, *colour_b;
   uint32_t *final_r, *final_g, *final_b, *final_w;
-  uint8_t *codes;
-  uint32_t *values;
 };
 
 struct StepParams {
   WaveState s;
   const uint32_t *in_queue;
-  uint32_t n;
   const uint16_t *bases;
   uint32_t B;
   const uint4 *blocks;
@@ -54,8 +51,6 @@ struct StepParams {
   uint32_t n_usages;
   uint32_t tick;
   float dof0, dof1;
-  uint8_t *codes;
-  uint32_t *values;
   svo_child_request *req_staging;
 };
 
@@ -85,23 +80,29 @@ struct DrawParams {
   uint32_t W, gsx, gsy;
 };
 
+// How a step's n work-items go to their queues, in work-item order.
 struct AppendParams {
-  const uint8_t *codes;
-  const uint32_t *values;
+  uint8_t *codes;    // per item: its queue and whether it requests a child
+  uint32_t *values;  // per item: its cone
   uint32_t n;
   uint32_t *queue[4];
   uint32_t capacity[kAppendTargets];
   uint32_t *counter[kAppendTargets];
   const svo_child_request *req_staging;
   svo_child_request *requests;
-  uint32_t *counts;  // kAppendTargets per chunk
+  uint32_t *counts;  // kAppendTargets per 1024 items
+  uint32_t *from;    // kAppendTargets: the counters before the step
 };
 
-uint32_t append_chunks(uint32_t n);
-int launch_append(const AppendParams &p, hipStream_t s);
-int launch_init(const InitParams &p, hipStream_t s);
-int launch_base_step(const StepParams &p, hipStream_t s);
-int launch_block_step(const StepParams &p, hipStream_t s);
+// *host (pinned) = tag << 32 | *counter, then *counter = 0.
+int launch_take_counter(uint32_t *counter, unsigned long long *host, uint32_t tag, hipStream_t s);
+
+// Work-groups of a step of n items.
+inline uint32_t append_steps(uint32_t n) { return (uint32_t)(((uint64_t)n + 1023u) / 1024u); }
+// A step and its appends.
+int launch_init(const InitParams &p, const AppendParams &a, hipStream_t s);
+int launch_base_step(const StepParams &p, const AppendParams &a, hipStream_t s);
+int launch_block_step(const StepParams &p, const AppendParams &a, hipStream_t s);
 int launch_background(const ShadeParams &p, hipStream_t s);
 int launch_remainders(const ShadeParams &p, hipStream_t s);
 int launch_draw(const DrawParams &p, hipStream_t s);

@@ -68,7 +68,7 @@ int scratch_for(Context *ctx, uint32_t n, bool staging) {
   int rc;
   if ((rc = ensure_scratch(ctx->wave_codes, std::max<size_t>(n, 1)))) return rc;
   if ((rc = ensure_scratch(ctx->wave_values, std::max<size_t>(n, 1) * 4))) return rc;
-  if ((rc = ensure_scratch(ctx->wave_counts, (size_t)std::max(1u, append_chunks(n)) * kAppendTargets * 4))) return rc;
+  if ((rc = ensure_scratch(ctx->wave_counts, ((size_t)append_steps(n) + 1) * kAppendTargets * 4))) return rc;
   if (staging && (rc = ensure_scratch(ctx->wave_staging, std::max<size_t>(n, 1) * sizeof(svo_child_request)))) return rc;
   return SVO_OK;
 }
@@ -76,10 +76,11 @@ int scratch_for(Context *ctx, uint32_t n, bool staging) {
 AppendParams append_base(Context *ctx, uint32_t n) {
   AppendParams a;
   std::memset(&a, 0, sizeof a);
-  a.codes = (const uint8_t *)ctx->wave_codes->ptr;
-  a.values = (const uint32_t *)ctx->wave_values->ptr;
+  a.codes = (uint8_t *)ctx->wave_codes->ptr;
+  a.values = (uint32_t *)ctx->wave_values->ptr;
   a.n = n;
-  a.counts = (uint32_t *)ctx->wave_counts->ptr;
+  a.from = (uint32_t *)ctx->wave_counts->ptr;
+  a.counts = a.from + kAppendTargets;
   return a;
 }
 
@@ -153,13 +154,10 @@ int enqueue_init(Context *ctx, Resolver &r, uint32_t gsx, uint32_t gsy) {
   p.final_g = (uint32_t *)fg.ptr;
   p.final_b = (uint32_t *)fbb.ptr;
   p.final_w = (uint32_t *)fw.ptr;
-  p.codes = (uint8_t *)ctx->wave_codes->ptr;
-  p.values = (uint32_t *)ctx->wave_values->ptr;
-  if (launch_init(p, ctx->stream)) return hip_fail(hipGetLastError(), "init launch");
   AppendParams a = append_base(ctx, (uint32_t)items);
   set_queue(a, kQueueBase, bq, bqid);
   set_queue(a, kQueueBackground, gq, gqid);
-  if (launch_append(a, ctx->stream)) return hip_fail(hipGetLastError(), "init append");
+  if (launch_init(p, a, ctx->stream)) return hip_fail(hipGetLastError(), "init launch");
   return SVO_OK;
 }
 
@@ -196,7 +194,6 @@ int enqueue_step(Context *ctx, Resolver &r, uint32_t n, bool block) {
     return fail(SVO_ERR_BUFFER_TOO_SMALL, "runBaseTrace: Bases is smaller than PowSum(BaseDepth)");
   if ((rc = scratch_for(ctx, n, block))) return rc;
   p.in_queue = (const uint32_t *)inq.ptr;
-  p.n = n;
   p.bases = (const uint16_t *)bases.ptr;
   p.B = in.base_depth;
   p.blocks = (const uint4 *)blocks.ptr;
@@ -206,11 +203,7 @@ int enqueue_step(Context *ctx, Resolver &r, uint32_t n, bool block) {
   p.tick = in.tick;
   p.dof0 = in.dof[0];
   p.dof1 = in.dof[1];
-  p.codes = (uint8_t *)ctx->wave_codes->ptr;
-  p.values = (uint32_t *)ctx->wave_values->ptr;
   p.req_staging = block ? (svo_child_request *)ctx->wave_staging->ptr : nullptr;
-  if ((block ? launch_block_step(p, ctx->stream) : launch_base_step(p, ctx->stream)))
-    return hip_fail(hipGetLastError(), "trace step launch");
   AppendParams a = append_base(ctx, n);
   set_queue(a, kQueueBase, bq, bqid);
   set_queue(a, kQueueBlock, kq, kqid);
@@ -222,7 +215,8 @@ int enqueue_step(Context *ctx, Resolver &r, uint32_t n, bool block) {
     a.capacity[4] = reqs.ptr ? std::min<uint32_t>(count_of(reqs, sizeof(svo_child_request)), in.max_child_request_id) : 0u;
     a.counter[4] = (uint32_t *)reqid.ptr;
   }
-  if (launch_append(a, ctx->stream)) return hip_fail(hipGetLastError(), "trace step append");
+  if (block ? launch_block_step(p, a, ctx->stream) : launch_base_step(p, a, ctx->stream))
+    return hip_fail(hipGetLastError(), "trace step launch");
   return SVO_OK;
 }
 

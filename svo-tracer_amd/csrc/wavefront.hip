@@ -4,10 +4,15 @@
 // for callers that drive the frame loop from the host through svo_enqueue
 // exactly as MainWindow.RunWavefront does (MainWindow.cs:356-622).
 //
-// Queue appends are deterministic and order-preserving: a step kernel writes one
-// code byte per work-item, then a count / scan / scatter pipeline appends the
-// items to their queues in work-item order (the reference's work-group atomic
-// `increment`, wavefront.cl:249-287, leaves the order to the scheduler).
+// Queue appends are deterministic and order-preserving (the reference's work-group atomic
+// `increment`, wavefront.cl:249-287, leaves the order to the scheduler): a step's
+// work-group of 1024 items counts its entries for each queue and either appends them
+// itself (a step of one work-group) or leaves a code byte per item and its counts to
+// append_kernel, whose work-groups sum the counts before their own.  A frame of the host
+// loop is some 770 steps, most of a few thousand items at its end, so a step is bound by its
+// launches: one or two instead of four, with coalesced appends (a thread that walked 16
+// consecutive items took 12.9 us a launch), made the appends of the 1080p depth-12 loop
+// 15.3 -> 1.7 ms of kernel time a frame and the frame 27 -> 18 ms (the host calls included).
 #include <hip/hip_runtime.h>
 
 #include "svo_device.hpp"
@@ -20,8 +25,7 @@ using namespace dev;
 namespace {
 
 constexpr uint32_t kThreads = 256;
-constexpr uint32_t kPerThread = 16;
-constexpr uint32_t kChunk = kThreads * kPerThread;
+constexpr uint32_t kStep = 1024;           // items of a step's work-group, one a thread
 
 __device__ __forceinline__ void load_state(const WaveState &s, uint32_t id, float o[3], float d[3], float &fov,
                                            uint64_t &x, uint64_t &y, uint64_t &z, uint32_t &depth) {
@@ -55,53 +59,41 @@ __device__ __forceinline__ uint32_t walk_address(const uint4 *blocks, uint32_t n
   return a;
 }
 
-// init, wavefront.cl:1352-1398
-__global__ void __launch_bounds__(kThreads) init_kernel(InitParams p) {
-  const uint32_t gx = blockIdx.x * kThreads + threadIdx.x;
-  const uint32_t gy = blockIdx.y;
-  uint8_t code = kCodeNone;
-  const uint32_t item = gx + gy * p.gsx;
-  if (gx < p.gsx && gy < p.gsy) {
-    const uint32_t id = gx + gy * p.W;
-    const uint32_t x = gx, y = gy;
-    if (id < p.s.n_rays && x < p.W && y < p.H) {
-      const float cu = p.lut[x], su = p.lut[p.W + x], cv = p.lut[2u * p.W + y], sv = p.lut[2u * p.W + p.H + y];
-      const float m0 = cu * cv, m1 = (0.0f - su) * cv, m2 = sv;
-      float d[3], inv[3];
-      for (int a = 0; a < 3; a++) {
-        d[a] = (p.facing[a] * m0 + p.facing[3 + a] * m1) + p.facing[6 + a] * m2;
-        inv[a] = 1.0f / d[a];
-      }
-      const float o[3] = {p.origin[0], p.origin[1], p.origin[2]};
-      uint64_t lx = 0, ly = 0, lz = 0;
-      const bool hit = trace_into_volume(o, d, inv, p.cone_fov, lx, ly, lz);
-      if (hit) store_loc(p.s, id, lx, ly, lz, 1u);
-      code = hit ? kQueueBase : kQueueBackground;
-      p.s.origins[id] = make_float4(o[0], o[1], o[2], 0.0f);
-      p.s.directions[id] = make_float4(d[0], d[1], d[2], 0.0f);
-      p.s.fovs[id] = p.cone_fov;
-      p.s.parents[id] = id;
-      p.s.weightings[id] = 255;
-      if (p.colour_r) p.colour_r[id] = 0;
-      if (p.colour_g) p.colour_g[id] = 0;
-      if (p.colour_b) p.colour_b[id] = 0;
-      p.final_r[id] = 0;
-      p.final_g[id] = 0;
-      p.final_b[id] = 0;
-      p.final_w[id] = 0;
-      p.values[item] = id;
-    }
+// init, wavefront.cl:1352-1398: the code of work-item (gx, gy); id is the cone it names.
+__device__ __forceinline__ uint8_t init_item(const InitParams &p, uint32_t item, uint32_t &id) {
+  const uint32_t gx = item % p.gsx, gy = item / p.gsx;
+  id = gx + gy * p.W;
+  if (id >= p.s.n_rays || gx >= p.W || gy >= p.H) return kCodeNone;
+  const float cu = p.lut[gx], su = p.lut[p.W + gx], cv = p.lut[2u * p.W + gy], sv = p.lut[2u * p.W + p.H + gy];
+  const float m0 = cu * cv, m1 = (0.0f - su) * cv, m2 = sv;
+  float d[3], inv[3];
+  for (int a = 0; a < 3; a++) {
+    d[a] = (p.facing[a] * m0 + p.facing[3 + a] * m1) + p.facing[6 + a] * m2;
+    inv[a] = 1.0f / d[a];
   }
-  if (gx < p.gsx && gy < p.gsy) p.codes[item] = code;
+  const float o[3] = {p.origin[0], p.origin[1], p.origin[2]};
+  uint64_t lx = 0, ly = 0, lz = 0;
+  const bool hit = trace_into_volume(o, d, inv, p.cone_fov, lx, ly, lz);
+  if (hit) store_loc(p.s, id, lx, ly, lz, 1u);
+  p.s.origins[id] = make_float4(o[0], o[1], o[2], 0.0f);
+  p.s.directions[id] = make_float4(d[0], d[1], d[2], 0.0f);
+  p.s.fovs[id] = p.cone_fov;
+  p.s.parents[id] = id;
+  p.s.weightings[id] = 255;
+  if (p.colour_r) p.colour_r[id] = 0;
+  if (p.colour_g) p.colour_g[id] = 0;
+  if (p.colour_b) p.colour_b[id] = 0;
+  p.final_r[id] = 0;
+  p.final_g[id] = 0;
+  p.final_b[id] = 0;
+  p.final_w[id] = 0;
+  return hit ? kQueueBase : kQueueBackground;
 }
 
 // runBaseTrace, wavefront.cl:1400-1463
-__global__ void __launch_bounds__(kThreads) base_step_kernel(StepParams p) {
-  const uint32_t i = blockIdx.x * kThreads + threadIdx.x;
-  if (i >= p.n) return;
+__device__ __forceinline__ uint8_t base_item(const StepParams &p, uint32_t i, uint32_t &id) {
   uint8_t code = kCodeNone;
-  const uint32_t id = p.in_queue[i];
-  p.values[i] = id;
+  id = p.in_queue[i];
   if (id < p.s.n_rays) {
     float o[3], d[3], fov;
     uint64_t x, y, z;
@@ -134,16 +126,13 @@ __global__ void __launch_bounds__(kThreads) base_step_kernel(StepParams p) {
       store_loc(p.s, id, x, y, z, depth);
     }
   }
-  p.codes[i] = code;
+  return code;
 }
 
 // runBlockTrace, wavefront.cl:1465-1566
-__global__ void __launch_bounds__(kThreads) block_step_kernel(StepParams p) {
-  const uint32_t i = blockIdx.x * kThreads + threadIdx.x;
-  if (i >= p.n) return;
+__device__ __forceinline__ uint8_t block_item(const StepParams &p, uint32_t i, uint32_t &id) {
   uint8_t code = kCodeNone;
-  const uint32_t id = p.in_queue[i];
-  p.values[i] = id;
+  id = p.in_queue[i];
   if (id < p.s.n_rays) {
     float o[3], d[3], fov;
     uint64_t x, y, z;
@@ -208,7 +197,89 @@ __global__ void __launch_bounds__(kThreads) block_step_kernel(StepParams p) {
       store_loc(p.s, id, x, y, z, depth);
     }
   }
-  p.codes[i] = code;
+  return code;
+}
+
+// Whether an item with code c goes to target t (a queue, or the child requests).
+__device__ __forceinline__ bool goes_to(uint8_t c, uint32_t t) {
+  return t < 4u ? (c & 7u) == t : c != kCodeNone && (c & kCodeRequest) != 0u;
+}
+
+__device__ __forceinline__ uint32_t lanes_below(uint64_t m) {
+  return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+}
+
+// Appends one wave's items (a lane each) behind pos[], which then counts them.
+__device__ __forceinline__ void append_wave(const AppendParams &a, uint8_t c, uint32_t value, uint32_t staged,
+                                            uint32_t pos[kAppendTargets]) {
+#pragma unroll
+  for (uint32_t t = 0; t < kAppendTargets; t++) {
+    const bool in = goes_to(c, t);
+    const uint64_t m = __ballot(in);
+    const uint32_t at = pos[t] + lanes_below(m);
+    if (in && at < a.capacity[t]) {
+      if (t < 4u) {
+        if (a.queue[t]) a.queue[t][at] = value;
+      } else if (a.requests) {
+        a.requests[at] = a.req_staging[staged];
+      }
+    }
+    pos[t] += (uint32_t)__popcll(m);
+  }
+}
+
+// One step (init, runBaseTrace or runBlockTrace) of 1024 work-items a work-group.  ONE: the step is
+// one work-group, which appends its items and moves the counters itself.
+enum { kInit, kBase, kBlock };
+template <int KIND, bool ONE, class Params>
+__global__ void __launch_bounds__(kStep) step_kernel(Params p, AppendParams a) {
+  __shared__ uint32_t s_count[kAppendTargets][kStep / 64], s_from[kAppendTargets];
+  const uint32_t i = blockIdx.x * kStep + threadIdx.x, lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+  uint8_t code = kCodeNone;
+  uint32_t id = 0;
+  if (i < a.n) {
+    if constexpr (KIND == kInit)
+      code = init_item(p, i, id);
+    else if constexpr (KIND == kBase)
+      code = base_item(p, i, id);
+    else
+      code = block_item(p, i, id);
+    if (!ONE) {
+      a.codes[i] = code;
+      a.values[i] = id;
+    }
+  }
+#pragma unroll
+  for (uint32_t t = 0; t < kAppendTargets; t++) {
+    const uint32_t c = (uint32_t)__popcll(__ballot(goes_to(code, t)));
+    if (lane == 0u) s_count[t][wave] = c;
+  }
+  // where the step's entries go: behind what each queue holds
+  if (blockIdx.x == 0 && threadIdx.x < kAppendTargets)
+    s_from[threadIdx.x] = a.counter[threadIdx.x] ? *a.counter[threadIdx.x] : 0u;
+  __syncthreads();
+  if (threadIdx.x < kAppendTargets) {
+    const uint32_t t = threadIdx.x;
+    uint32_t all = 0;
+    for (uint32_t w = 0; w < kStep / 64u; w++) {
+      const uint32_t c = s_count[t][w];
+      if (ONE) s_count[t][w] = s_from[t] + all;
+      all += c;
+    }
+    if (!ONE) {
+      if (blockIdx.x == 0) a.from[t] = s_from[t];
+      a.counts[kAppendTargets * blockIdx.x + t] = all;
+    } else if (a.counter[t]) {
+      *a.counter[t] = s_from[t] + all;
+    }
+  }
+  if (ONE) {
+    __syncthreads();
+    uint32_t pos[kAppendTargets];
+#pragma unroll
+    for (uint32_t t = 0; t < kAppendTargets; t++) pos[t] = s_count[t][wave];
+    append_wave(a, code, id, i, pos);
+  }
 }
 
 // evaluateBackground, wavefront.cl:1741-1797 (the light mix of non-primary cones
@@ -293,123 +364,122 @@ __global__ void __launch_bounds__(kThreads) draw_kernel(DrawParams p) {
   p.out[id] = c;
 }
 
-// ---- order-preserving append: count / scan / scatter ----
+// ---- order-preserving append of a step of several work-groups ----
 
-__device__ __forceinline__ void code_counts(uint8_t c, uint32_t v[kAppendTargets]) {
-  const uint32_t q = c & 7u;
-  for (uint32_t t = 0; t < 4; t++) v[t] += (q == t) ? 1u : 0u;
-  v[4] += (c != kCodeNone && (c & kCodeRequest)) ? 1u : 0u;
+// For steps of more than kSummed work-groups: exclusive sums of their counts, in place.  One
+// work-group; thread t sums a run of them.
+constexpr uint32_t kSummed = 4096;
+__global__ void __launch_bounds__(kThreads) append_scan_kernel(uint32_t *counts, uint32_t steps) {
+  __shared__ uint32_t s_run[kThreads];
+  const uint32_t per = (steps + kThreads - 1u) / kThreads;
+  const uint32_t b = min(steps, threadIdx.x * per), e = min(steps, b + per);
+  for (uint32_t t = 0; t < kAppendTargets; t++) {
+    uint32_t v = 0;
+    for (uint32_t k = b; k < e; k++) v += counts[kAppendTargets * k + t];
+    __syncthreads();
+    s_run[threadIdx.x] = v;
+    __syncthreads();
+    uint32_t before = 0;
+    for (uint32_t w = 0; w < threadIdx.x; w++) before += s_run[w];
+    for (uint32_t k = b; k < e; k++) {
+      const uint32_t c = counts[kAppendTargets * k + t];
+      counts[kAppendTargets * k + t] = before;
+      before += c;
+    }
+  }
 }
 
-__device__ void block_scan(uint32_t v[kAppendTargets], uint32_t total[kAppendTargets]) {
-  __shared__ uint32_t s_wave[kAppendTargets][kThreads / 64];
-  const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-  uint32_t incl[kAppendTargets];
-  for (int c = 0; c < kAppendTargets; c++) incl[c] = v[c];
-  for (int c = 0; c < kAppendTargets; c++)
-    for (int off = 1; off < 64; off <<= 1) {
-      const uint32_t t = __shfl_up(incl[c], off);
-      if (lane >= (uint32_t)off) incl[c] += t;
+// Work-group b appends the items of step work-group b: wave w its items 256w.., 64 consecutive ones a
+// round, so queue and request writes are coalesced, with all four rounds' loads in flight together.
+// summed: counts holds each step work-group's own counts, and those before b are summed here;
+// otherwise their exclusive sums.  The last work-group moves the counters (which nothing else
+// reads: a.from holds what they were).
+__global__ void __launch_bounds__(kThreads) append_kernel(AppendParams a, uint32_t summed) {
+  constexpr uint32_t kRounds = kStep / kThreads;
+  __shared__ uint32_t s_before[kAppendTargets][kThreads / 64], s_own[kAppendTargets][kThreads / 64];
+  const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, first = blockIdx.x * kStep + wave * 64u * kRounds;
+  uint8_t code[kRounds];
+  uint32_t value[kRounds];
+#pragma unroll
+  for (uint32_t r = 0; r < kRounds; r++) {
+    const uint32_t i = first + r * 64u + lane;
+    code[r] = i < a.n ? a.codes[i] : kCodeNone;
+    value[r] = i < a.n ? a.values[i] : 0u;
+  }
+  uint32_t before[kAppendTargets] = {0, 0, 0, 0, 0};
+  if (summed) {
+    for (uint32_t k = threadIdx.x; k < blockIdx.x; k += kThreads)
+#pragma unroll
+      for (uint32_t t = 0; t < kAppendTargets; t++) before[t] += a.counts[kAppendTargets * k + t];
+#pragma unroll
+    for (uint32_t t = 0; t < kAppendTargets; t++)
+      for (int off = 32; off > 0; off >>= 1) before[t] += __shfl_xor(before[t], off);
+  } else if (threadIdx.x == 0) {
+#pragma unroll
+    for (uint32_t t = 0; t < kAppendTargets; t++) before[t] = a.counts[kAppendTargets * blockIdx.x + t];
+  }
+#pragma unroll
+  for (uint32_t t = 0; t < kAppendTargets; t++) {
+    uint32_t own = 0;
+#pragma unroll
+    for (uint32_t r = 0; r < kRounds; r++) own += (uint32_t)__popcll(__ballot(goes_to(code[r], t)));
+    if (lane == 0u) {
+      s_before[t][wave] = before[t];
+      s_own[t][wave] = own;
     }
-  if (lane == 63u)
-    for (int c = 0; c < kAppendTargets; c++) s_wave[c][wave] = incl[c];
-  __syncthreads();
-  for (int c = 0; c < kAppendTargets; c++) {
-    uint32_t before = 0, all = 0;
-    for (uint32_t w = 0; w < kThreads / 64; w++) {
-      if (w < wave) before += s_wave[c][w];
-      all += s_wave[c][w];
-    }
-    v[c] = before + incl[c] - v[c];
-    total[c] = all;
   }
   __syncthreads();
-}
-
-__global__ void __launch_bounds__(kThreads) append_count_kernel(AppendParams p) {
-  const uint32_t base = blockIdx.x * kChunk + threadIdx.x * kPerThread;
-  uint32_t v[kAppendTargets] = {0, 0, 0, 0, 0};
-  for (uint32_t k = 0; k < kPerThread; k++)
-    if (base + k < p.n) code_counts(p.codes[base + k], v);
-  uint32_t total[kAppendTargets];
-  block_scan(v, total);
-  if (threadIdx.x == 0)
-    for (int c = 0; c < kAppendTargets; c++) p.counts[kAppendTargets * blockIdx.x + c] = total[c];
-}
-
-__global__ void __launch_bounds__(kThreads) append_scan_kernel(AppendParams p, uint32_t chunks) {
-  uint32_t carry[kAppendTargets];
-  for (int c = 0; c < kAppendTargets; c++) carry[c] = p.counter[c] ? *p.counter[c] : 0u;
-  __syncthreads();
-  for (uint32_t start = 0; start < chunks; start += kThreads) {
-    const uint32_t i = start + threadIdx.x;
-    uint32_t v[kAppendTargets] = {0, 0, 0, 0, 0};
-    if (i < chunks)
-      for (int c = 0; c < kAppendTargets; c++) v[c] = p.counts[kAppendTargets * i + c];
-    uint32_t total[kAppendTargets];
-    block_scan(v, total);
-    if (i < chunks)
-      for (int c = 0; c < kAppendTargets; c++) p.counts[kAppendTargets * i + c] = carry[c] + v[c];
-    for (int c = 0; c < kAppendTargets; c++) carry[c] += total[c];
-  }
-  __syncthreads();
-  if (threadIdx.x == 0)
-    for (int c = 0; c < kAppendTargets; c++)
-      if (p.counter[c]) *p.counter[c] = carry[c];
-}
-
-__global__ void __launch_bounds__(kThreads) append_scatter_kernel(AppendParams p) {
-  const uint32_t base = blockIdx.x * kChunk + threadIdx.x * kPerThread;
-  uint32_t v[kAppendTargets] = {0, 0, 0, 0, 0};
-  for (uint32_t k = 0; k < kPerThread; k++)
-    if (base + k < p.n) code_counts(p.codes[base + k], v);
-  uint32_t total[kAppendTargets];
-  block_scan(v, total);
   uint32_t pos[kAppendTargets];
-  for (int c = 0; c < kAppendTargets; c++) pos[c] = p.counts[kAppendTargets * blockIdx.x + c] + v[c];
-  for (uint32_t k = 0; k < kPerThread; k++) {
-    const uint32_t i = base + k;
-    if (i >= p.n) break;
-    const uint8_t c = p.codes[i];
-    if (c == kCodeNone) continue;
-    const uint32_t q = c & 7u;
-    if (q < 4u) {
-      if (p.queue[q] && pos[q] < p.capacity[q]) p.queue[q][pos[q]] = p.values[i];
-      pos[q]++;
-    }
-    if (c & kCodeRequest) {
-      if (p.requests && pos[4] < p.capacity[4]) p.requests[pos[4]] = p.req_staging[i];
-      pos[4]++;
-    }
+#pragma unroll
+  for (uint32_t t = 0; t < kAppendTargets; t++) {
+    pos[t] = a.from[t];
+    for (uint32_t w = 0; w < kThreads / 64u; w++) pos[t] += s_before[t][w] + (w < wave ? s_own[t][w] : 0u);
   }
+#pragma unroll
+  for (uint32_t r = 0; r < kRounds; r++) append_wave(a, code[r], value[r], first + r * 64u + lane, pos);
+  if (blockIdx.x == gridDim.x - 1u && threadIdx.x == kThreads - 1u) {
+#pragma unroll
+    for (uint32_t t = 0; t < kAppendTargets; t++)
+      if (a.counter[t]) *a.counter[t] = pos[t];
+  }
+}
+
+// ResetIDBuffer's device half: the counter goes to pinned host memory, tagged with the call's
+// number, and is cleared.
+__global__ void take_counter_kernel(uint32_t *counter, unsigned long long *host, uint32_t tag) {
+  const uint32_t v = *counter;
+  *counter = 0u;
+  __hip_atomic_store(host, ((unsigned long long)tag << 32) | v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+template <int KIND, class Params>
+int launch_step(const Params &p, const AppendParams &a, hipStream_t s) {
+  if (a.n == 0u) return 0;
+  const uint32_t steps = append_steps(a.n);
+  if (steps == 1u) {
+    hipLaunchKernelGGL((step_kernel<KIND, true, Params>), dim3(1), dim3(kStep), 0, s, p, a);
+    return hipGetLastError() == hipSuccess ? 0 : -1;
+  }
+  hipLaunchKernelGGL((step_kernel<KIND, false, Params>), dim3(steps), dim3(kStep), 0, s, p, a);
+  if (hipGetLastError() != hipSuccess) return -1;
+  if (steps > kSummed) hipLaunchKernelGGL(append_scan_kernel, dim3(1), dim3(kThreads), 0, s, a.counts, steps);
+  hipLaunchKernelGGL(append_kernel, dim3(steps), dim3(kThreads), 0, s, a, steps > kSummed ? 0u : 1u);
+  return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
 }  // namespace
 
-uint32_t append_chunks(uint32_t n) { return (n + kChunk - 1u) / kChunk; }
-
-int launch_append(const AppendParams &p, hipStream_t s) {
-  const uint32_t chunks = append_chunks(p.n);
-  if (chunks == 0) return 0;
-  hipLaunchKernelGGL(append_count_kernel, dim3(chunks), dim3(kThreads), 0, s, p);
-  hipLaunchKernelGGL(append_scan_kernel, dim3(1), dim3(kThreads), 0, s, p, chunks);
-  hipLaunchKernelGGL(append_scatter_kernel, dim3(chunks), dim3(kThreads), 0, s, p);
+int launch_take_counter(uint32_t *counter, unsigned long long *host, uint32_t tag, hipStream_t s) {
+  hipLaunchKernelGGL(take_counter_kernel, dim3(1), dim3(1), 0, s, counter, host, tag);
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
-int launch_init(const InitParams &p, hipStream_t s) {
-  hipLaunchKernelGGL(init_kernel, dim3((p.gsx + kThreads - 1) / kThreads, p.gsy), dim3(kThreads), 0, s, p);
-  return hipGetLastError() == hipSuccess ? 0 : -1;
-}
+int launch_init(const InitParams &p, const AppendParams &a, hipStream_t s) { return launch_step<kInit>(p, a, s); }
 
-int launch_base_step(const StepParams &p, hipStream_t s) {
-  hipLaunchKernelGGL(base_step_kernel, dim3((p.n + kThreads - 1) / kThreads), dim3(kThreads), 0, s, p);
-  return hipGetLastError() == hipSuccess ? 0 : -1;
-}
+int launch_base_step(const StepParams &p, const AppendParams &a, hipStream_t s) { return launch_step<kBase>(p, a, s); }
 
-int launch_block_step(const StepParams &p, hipStream_t s) {
-  hipLaunchKernelGGL(block_step_kernel, dim3((p.n + kThreads - 1) / kThreads), dim3(kThreads), 0, s, p);
-  return hipGetLastError() == hipSuccess ? 0 : -1;
+int launch_block_step(const StepParams &p, const AppendParams &a, hipStream_t s) {
+  return launch_step<kBlock>(p, a, s);
 }
 
 int launch_background(const ShadeParams &p, hipStream_t s) {
