@@ -449,10 +449,10 @@ extern "C" int svo_stream_update(svo_context *ctx, const svo_terrain *t, const s
   // the free groups, then every counter of the update in one read
   if ((rc = st.count_into(pv.usages, 0, pv.n_usages, kSelFree, state + kShFree))) return rc;
   uint32_t *host = ctx->stream_host;
-  hipError_t e = hipMemcpyAsync(host, state, kShSlots * 4, hipMemcpyDeviceToHost, s);
-  if (e == hipSuccess && tree_counters)
-    e = hipMemcpyAsync(host + kShSlots, tree_counters, kTcSlots * 4, hipMemcpyDeviceToHost, s);
-  if (e == hipSuccess) e = hipStreamSynchronize(s);
+  if ((rc = st.launch(launch_tell(state, kShSlots, tree_counters, tree_counters ? kTcSlots : 0u, host, nullptr, 0, s),
+                      "counter read")))
+    return rc;
+  hipError_t e = hipStreamSynchronize(s);
   if (e != hipSuccess) return hip_fail(e, "svo_stream_update: counter read");
   out.requests = stored ? host[kShRequests] : 0u;
   out.unique = host[kShUnique];

@@ -77,7 +77,7 @@ struct FrameParams {
   uint32_t lanes;  // lanes of a wave that take cones, a power of two (64: all)
   uint32_t chunk;  // work items a wave claims per atomic (multiple of 64)
   // tile schedule (may be null): position k of a band's work range holds tile order[k]; a
-  // wave stores the loop iterations it spent on a tile in tile_cost[tile]
+  // wave stores the most steps any of a tile's cones took in tile_cost[tile]
   const uint32_t *order;
   uint32_t *tile_cost;
 };

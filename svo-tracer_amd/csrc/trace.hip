@@ -687,8 +687,8 @@ trace_frame_kernel(const FrameParams p) {
 
 // ---- tile schedule ----
 
-// Cost class of a tile: floor(log2(iterations)) - 2, clamped to 0..kCostClasses-1 (tiles of
-// fewer than 8 iterations, and unmeasured ones, are class 0; 512 and more, class 7).
+// Cost class of a tile: floor(log2(steps of its longest cone)) - 2, clamped to 0..kCostClasses-1 (tiles of
+// fewer than 8 steps, and unmeasured ones, are class 0; 512 and more, class 7).
 constexpr uint32_t kCostClasses = 8;
 __device__ __forceinline__ uint32_t cost_class(uint32_t c) {
   const uint32_t l = c ? 31u - (uint32_t)__clz(c) : 0u;

@@ -3,8 +3,11 @@
 //
 // Every phase runs on the device and sizes itself from device-side counts; the host sequences
 // the kernels and reads the counters back once at the end of a dispatch, once per collection
-// pass, and once per free walk that has not ended within its first kSpecLevels levels (each
-// level reads its frontier size on the device, so the first levels are launched unread).
+// pass, once for the groups of grafts whose records it has not seen, and again for a free walk
+// that has not ended within its first kSpecLevels levels (each level reads its frontier size on
+// the device; what follows the walk is launched with it and does nothing while it is not over).
+// A prune and a graft of 4096 records: 52 launches, 6 uploads and 6 waits -> 27 launches and 3
+// waits.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -86,7 +89,7 @@ struct Op {
   Context *ctx;
   PoolView pv{};
   TreeScratch ts{};
-  uint32_t *host = nullptr;  // pinned counter mirror
+  uint32_t *host = nullptr;  // pinned counter mirror; the word behind it is the last read's tag
 
   std::shared_ptr<DeviceBuffer> &buf(int k) { return ctx->tree_scratch[k]; }
 
@@ -118,8 +121,9 @@ struct Op {
     pv.B = in.base_depth;
     pv.now = in.tick;
     if (!ctx->tree_host) {
-      hipError_t e = hipHostMalloc((void **)&ctx->tree_host, kTcSlots * sizeof(uint32_t), hipHostMallocDefault);
+      hipError_t e = hipHostMalloc((void **)&ctx->tree_host, (kTcSlots + 1) * sizeof(uint32_t), hipHostMallocDefault);
       if (e != hipSuccess) return hip_fail(e, "hipHostMalloc");
+      ctx->tree_host[kTcSlots] = 0;
     }
     host = ctx->tree_host;
     void *p;
@@ -141,10 +145,10 @@ struct Op {
     ts.claimed = (uint32_t *)p;
     if ((rc = grow(kTbChunks, ((size_t)pv.n_usages / kCollectChunk + 2) * 4, &p))) return rc;
     ts.chunk_counts = (uint32_t *)p;
-    if ((rc = context_scan_sums(ctx, scan_span_sums_bytes(pv.n_usages / kCollectChunk + 1), &ts.scan_sums)))
-      return rc;
-    return tree_fill_u32(ts.counters, 0, kTcSlots, ctx->stream) ? fail(SVO_ERR_HIP, "tree: fill") : SVO_OK;
+    return context_scan_sums(ctx, scan_span_sums_bytes(pv.n_usages / kCollectChunk + 1), &ts.scan_sums);
   }
+  // The dispatch's first launch, once its buffers are there.
+  int begin() { return launch(launch_begin(ts, ctx->stream), "begin"); }
 
   int records(uint32_t n, uint32_t table_entries) {
     void *p;
@@ -157,35 +161,57 @@ struct Op {
     if ((rc = grow(kTbVals, (size_t)cap * 4, &p))) return rc;
     ts.vals = (uint32_t *)p;
     ts.table_mask = cap - 1u;
-    if (tree_fill_u64(ts.keys, ~0ull, cap, ctx->stream) || tree_fill_u32(ts.vals, 0, cap, ctx->stream))
-      return fail(SVO_ERR_HIP, "tree: fill");
     return SVO_OK;
   }
 
-  // Reads counter slots [first, first+count) into host[first...].
-  int read(uint32_t first, uint32_t count) {
-    hipError_t e = hipMemcpyAsync(host + first, ts.counters + first, count * 4, hipMemcpyDeviceToHost, ctx->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
+  // The counter block into `host` and a stream wait.
+  int read() {
+    if (launch_tell(ts.counters, kTcSlots, nullptr, 0, host, nullptr, 0, ctx->stream))
+      return fail(SVO_ERR_HIP, "tree: counter read");
+    const hipError_t e = hipStreamSynchronize(ctx->stream);
     return e == hipSuccess ? SVO_OK : hip_fail(e, "tree: counter read");
+  }
+  // The same in the middle of a dispatch: the host watches the tag behind the words instead of
+  // waiting for the stream (25 us -> 10 us until the next kernel starts).  Should the tag not
+  // arrive, the stream's state decides.
+  int peek() {
+    uint32_t *word = host + kTcSlots;
+    const uint32_t tag = *word + 1u;
+    if (launch_tell(ts.counters, kTcSlots, nullptr, 0, host, word, tag, ctx->stream))
+      return fail(SVO_ERR_HIP, "tree: counter read");
+    for (uint32_t spins = 1; __atomic_load_n(word, __ATOMIC_ACQUIRE) != tag; spins++) {
+      if (spins % (1u << 20)) continue;
+      const hipError_t e = hipStreamQuery(ctx->stream);
+      if (e == hipErrorNotReady) continue;
+      if (e != hipSuccess) return hip_fail(e, "tree: counter read");
+      if (__atomic_load_n(word, __ATOMIC_ACQUIRE) != tag) return fail(SVO_ERR_HIP, "tree: the counters did not arrive");
+      break;
+    }
+    return SVO_OK;
   }
 
   int launch(int r, const char *what) { return r ? fail(SVO_ERR_HIP, std::string("tree: launch ") + what) : SVO_OK; }
 
   // Frees the subtrees queued in front[0] (count in its counter), level by level, then
-  // applies the multi-parent unlink events in order.  The first kSpecLevels levels are
-  // launched without reading anything back; with `finish_walk` the host then reads the
-  // frontier and adds levels until it is empty.  Without it (a walk known to end within those
-  // levels) an unfinished walk is flagged on the device, as are overflows of the frontier or
-  // of the event table, and finish() reports them.
-  int free_walk(bool use_stop, bool finish_walk = true) {
+  // applies the multi-parent unlink events in order and launches `after`, which does nothing while
+  // the walk is pending.  The first kSpecLevels levels and what follows go out without reading
+  // anything back; then the host reads the counters (with `last` it waits for the stream) and, if
+  // the walk is pending, adds levels until it is over and launches the rest again.  With
+  // read_back false (a walk known to end within those levels) an unfinished walk is flagged on the
+  // device, as are overflows of the frontier or of the event table, for the caller's read.
+  template <class After>
+  int free_walk(bool use_stop, const RecordFields &f, uint32_t n_records, const uint64_t *locs, bool read_back,
+                bool last, After after) {
     int rc = walk_levels(use_stop, 0, kSpecLevels);
-    if (rc) return rc;
+    if (!rc) rc = launch(launch_unlink(pv, ts, kSpecLevels, read_back, f, n_records, locs, ctx->stream), "unlink");
+    if (!rc) rc = after();
+    if (!rc && read_back) rc = last ? read() : peek();
+    if (rc || !read_back || !host[kTcPending]) return rc;
     uint32_t level = kSpecLevels;
-    if (finish_walk) {
-      if ((rc = read(front_slot(level % 3u), 1))) return rc;
-      if ((rc = walk_on(use_stop, &level))) return rc;
-    }
-    return end_walk(level);
+    if ((rc = walk_on(use_stop, &level))) return rc;
+    rc = launch(launch_unlink(pv, ts, level, false, f, 0, locs, ctx->stream), "unlink");
+    if (!rc) rc = after();
+    return rc ? rc : last ? read() : peek();
   }
   // After a read of the frontier of `*level`: while it is not empty, the next kMoreLevels
   // levels go out unread and the frontier after them is read (a walk that outlasts the
@@ -194,7 +220,7 @@ struct Op {
     while (*level < kMaxFreeLevels && host[front_slot(*level % 3u)] != 0) {
       const uint32_t to = std::min(*level + kMoreLevels, kMaxFreeLevels);
       int rc = walk_levels(use_stop, *level, to);
-      if (!rc) rc = read(front_slot(to % 3u), 1);
+      if (!rc) rc = peek();
       if (rc) return rc;
       *level = to;
     }
@@ -207,7 +233,6 @@ struct Op {
     }
     return SVO_OK;
   }
-  int end_walk(uint32_t levels) { return launch(launch_unlink(pv, ts, levels, ctx->stream), "unlink"); }
 
   // Collection (graft, wavefront.cl:1277-1305): up to `need` groups (at most need_max) into
   // ts.list; the count collected accumulates in counters[kTcGot].  One pass per age
@@ -220,23 +245,18 @@ struct Op {
     ts.list = (uint32_t *)p;
     ts.list_capacity = need_max;
     if (!need_max) return SVO_OK;
-    if ((rc = launch(tree_fill_u32(ts.claimed, 0, ts.claimed_words + 1, ctx->stream), "fill"))) return rc;
     uint32_t ng = pv.n_usages;
     if (in.memory_size) ng = (uint32_t)std::min<uint64_t>(((uint64_t)in.memory_size + 7u) / 8u, ng);
     for (uint32_t offset = in.offset;; offset >>= 1) {
       if ((rc = launch(launch_collect_count(pv, ng, offset, false, ts, ctx->stream), "collect count"))) return rc;
-      if ((rc = launch(launch_collect_limit(ts, need, ctx->stream), "collect limit"))) return rc;
-      if ((rc = launch(launch_collect_scatter(pv, ng, offset, false, ts, ctx->stream), "collect scatter"))) return rc;
+      if ((rc = launch(launch_collect_scatter(pv, ng, offset, false, need, ts, ctx->stream), "collect scatter")))
+        return rc;
       if ((rc = launch(launch_collect_claim(pv, need_max, ts, ctx->stream), "collect claim"))) return rc;
-      // the pass's groups count as collected now (mark and the next pass read kTcFrom / kTcK)
-      if ((rc = launch(launch_collect_advance(ts, ctx->stream), "collect advance"))) return rc;
-      if ((rc = walk_levels(true, 0, kSpecLevels))) return rc;
-      // one read: the walk's frontier, the groups collected so far and (device need) the need
-      if ((rc = read(0, kTcSlots))) return rc;
-      uint32_t level = kSpecLevels;
-      if ((rc = walk_on(true, &level))) return rc;
-      if ((rc = end_walk(level))) return rc;
-      if ((rc = launch(launch_collect_mark(pv, need_max, pv.now, ts, ctx->stream), "collect mark"))) return rc;
+      // its read: the walk's state, the groups collected so far and (device need) the need
+      rc = free_walk(true, RecordFields{}, 0, nullptr, true, false, [&] {
+        return launch(launch_collect_mark(pv, need_max, pv.now, ts, ctx->stream), "collect mark");
+      });
+      if (rc) return rc;
       const uint32_t nd = need.p ? std::min(host[kTcNeed], need.v) : need.v;
       if (offset == 0 || host[kTcGot] >= nd) break;
     }
@@ -247,35 +267,42 @@ struct Op {
   // parent, what hangs below it is freed and the group itself gets tick 0.
   int reclaim(const svo_update_input_data &in, uint32_t *got) {
     *got = 0;
-    int rc = launch(tree_fill_u32(ts.claimed, 0, ts.claimed_words + 1, ctx->stream), "fill");
+    int rc = begin();
     if (rc) return rc;
     uint32_t ng = pv.n_usages;
     if (in.memory_size) ng = (uint32_t)std::min<uint64_t>(((uint64_t)in.memory_size + 7u) / 8u, ng);
     if ((rc = launch(launch_collect_count(pv, ng, in.offset, true, ts, ctx->stream), "reclaim count"))) return rc;
-    if ((rc = read(kTcTotal, 1))) return rc;
+    if ((rc = peek())) return rc;
     const uint32_t k = host[kTcTotal];
     if (!k) return finish(nullptr);
     void *p;
     if ((rc = grow(kTbList, (size_t)k * 4, &p))) return rc;
     ts.list = (uint32_t *)p;
     ts.list_capacity = k;
-    if ((rc = launch(launch_collect_limit(ts, host_count(k), ctx->stream), "reclaim limit"))) return rc;
-    if ((rc = launch(launch_collect_scatter(pv, ng, in.offset, true, ts, ctx->stream), "reclaim scatter"))) return rc;
+    if ((rc = launch(launch_collect_scatter(pv, ng, in.offset, true, host_count(k), ts, ctx->stream),
+                     "reclaim scatter")))
+      return rc;
     if ((rc = launch(launch_collect_claim(pv, k, ts, ctx->stream), "reclaim claim"))) return rc;
-    if ((rc = free_walk(true))) return rc;
-    if ((rc = launch(launch_collect_mark(pv, k, 0u, ts, ctx->stream), "reclaim mark"))) return rc;
-    if ((rc = finish(nullptr))) return rc;
+    rc = free_walk(true, RecordFields{}, 0, nullptr, true, true,
+                   [&] { return launch(launch_collect_mark(pv, k, 0u, ts, ctx->stream), "reclaim mark"); });
+    if (!rc) rc = stats_from(host, nullptr);
+    if (rc) return rc;
     *got = k;
     return SVO_OK;
   }
 
   // Reads the counters once, reports a flagged overflow and fills `out` (may be null).
   int finish(svo_tree_stats *out) {
-    int rc = read(0, kTcSlots);
+    int rc = read();
     if (rc) return rc;
     return stats_from(host, out);
   }
 };
+
+// The depth and address words of a record array.
+RecordFields fields_of(const void *rec, size_t stride, size_t depth, size_t address) {
+  return RecordFields{(const uint8_t *)rec, (uint32_t)stride, (uint32_t)depth, (uint32_t)address};
+}
 
 int prune_impl(Context *ctx, const Pool &pool, const svo_update_input_data &in, const svo_pruning *rec, uint32_t n,
                const svo_block *surface, uint32_t n_surface, const uint64_t *locs, uint32_t n_locs,
@@ -288,26 +315,23 @@ int prune_impl(Context *ctx, const Pool &pool, const svo_update_input_data &in, 
   hipStream_t s = ctx->stream;
   const PoolView &pv = op.pv;
   const TreeScratch &ts = op.ts;
-  const uint8_t *rb = reinterpret_cast<const uint8_t *>(rec);
+  const RecordFields f =
+      fields_of(rec, sizeof(svo_pruning), offsetof(svo_pruning, depth), offsetof(svo_pruning, address));
+  if ((rc = op.begin())) return rc;
   if ((rc = op.launch(launch_prune_resolve(pv, rec, n, n_surface, locs, n_locs, ts, s), "prune resolve"))) return rc;
-  if ((rc = op.launch(launch_requests_and_touches(pv, rb + offsetof(svo_pruning, depth), sizeof(svo_pruning),
-                                                  reinterpret_cast<const uint32_t *>(rb + offsetof(svo_pruning, address)),
-                                                  sizeof(svo_pruning), n, locs, ts, s),
-                      "prune requests")))
-    return rc;
-  if ((rc = op.launch(launch_prune_winners(pv, rec, n, ts, s), "prune winners"))) return rc;
-  if ((rc = op.launch(launch_prune_roots(pv, rec, n, ts, s), "prune roots"))) return rc;
-  if ((rc = op.free_walk(false))) return rc;
-  if ((rc = op.launch(launch_prune_apply(pv, rec, n, surface, ts, s), "prune apply"))) return rc;
-  return op.finish(stats);
+  if ((rc = op.launch(launch_touches(pv, f, n, locs, ts, s), "prune touches"))) return rc;
+  rc = op.free_walk(false, f, n, locs, true, true,
+                    [&] { return op.launch(launch_prune_apply(pv, rec, n, surface, ts, s), "prune apply"); });
+  return rc ? rc : stats_from(op.host, stats);
 }
 
 // dev_records: when set, the number of records lives there on the device (at most n) and the
 // dispatch reads nothing back: its counters stay in the op's counter block for the caller
-// (graft_counters) to read with its own.
+// (graft_counters) to read with its own.  host_records: the records, where the host has them: it
+// then bounds the grafts' groups itself.
 int graft_impl(Context *ctx, const Pool &pool, const svo_update_input_data &in, const svo_grafting *rec, uint32_t n,
                const svo_block *gb, uint32_t n_gb, const uint64_t *locs, uint32_t n_locs, svo_tree_stats *stats,
-               const uint32_t *dev_records = nullptr) {
+               const uint32_t *dev_records = nullptr, const svo_grafting *host_records = nullptr) {
   Op op{ctx};
   int rc = op.init(pool, in);
   if (rc) return rc;
@@ -324,6 +348,7 @@ int graft_impl(Context *ctx, const Pool &pool, const svo_update_input_data &in, 
   op.ts.need = (uint32_t *)p;
   if ((rc = op.grow(kTbStart, per_rec, &p))) return rc;
   op.ts.start = (uint32_t *)p;
+  if ((rc = op.begin())) return rc;
   const DevCount records{n, dev_records};
   // structure: sizes, where each graft's numbering lives, pre-order numbering, needs
   if ((rc = op.launch(launch_graft_sizes(rec, records, n_gb, op.ts, s), "graft sizes"))) return rc;
@@ -331,11 +356,15 @@ int graft_impl(Context *ctx, const Pool &pool, const svo_update_input_data &in, 
   if ((rc = context_scan_sums(ctx, scan_span_sums_bytes(n), &sums))) return rc;
   if ((rc = op.launch(launch_scan_u32(op.ts.size, op.ts.where, n, op.ts.counters + kTcTotal, sums, s), "scan")))
     return rc;
-  // groups of all grafts: read back for host records; for device records every graft's
-  // groups lie in its own part of the graft blocks, so n_gb / 8 bounds them
+  // groups of all grafts: added up here for records the host has, read back for bound ones; for
+  // counted ones every graft's groups lie in its own part of the graft blocks, so n_gb / 8
+  // bounds them
   uint32_t groups = n_gb / 8u;
-  if (!dev_records) {
-    if ((rc = op.read(kTcTotal, 1))) return rc;
+  if (host_records) {
+    groups = 0;
+    for (uint32_t i = 0; i < n; i++) groups += graft_groups(host_records[i], n_gb);
+  } else if (!dev_records) {
+    if ((rc = op.peek())) return rc;
     groups = op.host[kTcTotal];
   }
   if ((rc = op.grow(kTbNumber, ((size_t)groups + 1) * 4, &p))) return rc;
@@ -351,22 +380,18 @@ int graft_impl(Context *ctx, const Pool &pool, const svo_update_input_data &in, 
   const DevCount got{groups, op.ts.counters + kTcGot};
   const PoolView &pv = op.pv;
   const TreeScratch &ts = op.ts;
-  const uint8_t *rb = reinterpret_cast<const uint8_t *>(rec);
-  if ((rc = op.launch(launch_graft_resolve(pv, rec, n, locs, n_locs, ts, s), "graft resolve"))) return rc;
-  if ((rc = op.launch(launch_requests_and_touches(pv, rb + offsetof(svo_grafting, depth), sizeof(svo_grafting),
-                                                  reinterpret_cast<const uint32_t *>(rb + offsetof(svo_grafting, graft_address)),
-                                                  sizeof(svo_grafting), n, locs, ts, s),
-                      "graft requests")))
-    return rc;
-  if ((rc = op.launch(launch_graft_winners(pv, n, got, ts, s), "graft winners"))) return rc;
-  if ((rc = op.launch(launch_graft_roots(pv, records, got, ts, s), "graft roots"))) return rc;
+  const RecordFields f =
+      fields_of(rec, sizeof(svo_grafting), offsetof(svo_grafting, depth), offsetof(svo_grafting, graft_address));
+  if ((rc = op.launch(launch_graft_resolve(pv, rec, n, locs, n_locs, got, ts, s), "graft resolve"))) return rc;
+  if ((rc = op.launch(launch_graft_roots(pv, f, records, locs, got, ts, s), "graft roots"))) return rc;
   // device records come from the streaming update, whose targets are childless blocks: their
   // walk is empty, and one that is not is flagged rather than read back and finished
-  if ((rc = op.free_walk(true, !dev_records))) return rc;
-  if ((rc = op.launch(launch_graft_place(pv, rec, n, need, gb, ts, s), "graft place"))) return rc;
-  if ((rc = op.launch(launch_graft_release(pv, n, got, ts, s), "graft release"))) return rc;
-  if (dev_records) return SVO_OK;
-  return op.finish(stats);
+  rc = op.free_walk(true, f, n, locs, !dev_records, true, [&] {
+    const int r = op.launch(launch_graft_place(pv, rec, n, need, gb, ts, s), "graft place");
+    return r ? r : op.launch(launch_graft_finish(pv, n, got, ts, s), "graft finish");
+  });
+  if (rc || dev_records) return rc;
+  return stats_from(op.host, stats);
 }
 
 Pool pool_from_context(Context *ctx) {
@@ -388,7 +413,9 @@ Pool pool_from_context(Context *ctx) {
   return p;
 }
 
-// Copies a host array into a context scratch buffer; returns its device address.
+// Copies a host array into a context scratch buffer; returns its device address.  The copy is not
+// waited for: a dispatch ends with a wait for its stream, which covers it (three waits took some
+// 45 us of a dispatch).
 int stage(Context *ctx, int slot, const void *src, size_t bytes, const void **out) {
   *out = nullptr;
   if (!bytes) return SVO_OK;
@@ -396,7 +423,6 @@ int stage(Context *ctx, int slot, const void *src, size_t bytes, const void **ou
   int rc = ensure_scratch(ctx->tree_scratch[slot], bytes);
   if (rc) return rc;
   hipError_t e = hipMemcpyAsync(ctx->tree_scratch[slot]->ptr, src, bytes, hipMemcpyHostToDevice, ctx->stream);
-  if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
   if (e != hipSuccess) return hip_fail(e, "tree management: upload");
   *out = ctx->tree_scratch[slot]->ptr;
   return SVO_OK;
@@ -510,9 +536,12 @@ extern "C" int svo_prune(svo_context *ctx, const svo_update_input_data *input, c
   int rc = stage(ctx, kTbRecords, records, (size_t)n * sizeof(svo_pruning), &d_rec);
   if (!rc) rc = stage(ctx, kTbSide, surface, (size_t)n_surface * sizeof(svo_block), &d_side);
   if (!rc) rc = stage(ctx, kTbLocations, locations, (size_t)n_locations * 24, &d_loc);
-  if (rc) return rc;
-  return prune_impl(ctx, pool_from_context(ctx), *input, (const svo_pruning *)d_rec, n, (const svo_block *)d_side,
+  if (!rc)
+    rc = prune_impl(ctx, pool_from_context(ctx), *input, (const svo_pruning *)d_rec, n, (const svo_block *)d_side,
                     n_surface, (const uint64_t *)d_loc, n_locations, stats);
+  // a call that failed early has not waited for its copies out of the caller's arrays
+  if (rc) (void)hipStreamSynchronize(ctx->stream);
+  return rc;
 }
 
 extern "C" int svo_graft(svo_context *ctx, const svo_update_input_data *input, const svo_grafting *records, uint32_t n,
@@ -524,9 +553,11 @@ extern "C" int svo_graft(svo_context *ctx, const svo_update_input_data *input, c
   int rc = stage(ctx, kTbRecords, records, (size_t)n * sizeof(svo_grafting), &d_rec);
   if (!rc) rc = stage(ctx, kTbSide, graft_blocks, (size_t)n_graft_blocks * sizeof(svo_block), &d_gb);
   if (!rc) rc = stage(ctx, kTbLocations, locations, (size_t)n_locations * 24, &d_loc);
-  if (rc) return rc;
-  return graft_impl(ctx, pool_from_context(ctx), *input, (const svo_grafting *)d_rec, n, (const svo_block *)d_gb,
-                    n_graft_blocks, (const uint64_t *)d_loc, n_locations, stats);
+  if (!rc)
+    rc = graft_impl(ctx, pool_from_context(ctx), *input, (const svo_grafting *)d_rec, n, (const svo_block *)d_gb,
+                    n_graft_blocks, (const uint64_t *)d_loc, n_locations, stats, nullptr, records);
+  if (rc) (void)hipStreamSynchronize(ctx->stream);  // as in svo_prune
+  return rc;
 }
 
 extern "C" int svo_reclaim(svo_context *ctx, const svo_update_input_data *input, uint32_t *reclaimed) {
@@ -545,6 +576,7 @@ extern "C" int svo_collect(svo_context *ctx, const svo_update_input_data *input,
   Op op{ctx};
   int rc = op.init(pool_from_context(ctx), *input);
   if (rc) return rc;
+  if ((rc = op.begin())) return rc;
   if ((rc = op.collect(*input, host_count(need), need))) return rc;
   if ((rc = op.finish(nullptr))) return rc;
   const uint32_t got = op.host[kTcGot];

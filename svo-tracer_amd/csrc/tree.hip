@@ -129,6 +129,21 @@ __device__ __forceinline__ void push(uint2 *front, uint32_t *count, uint32_t cap
     atomicOr(overflow, 1u);
 }
 
+// Queues the groups below group g's blocks: the eight Child words are loaded together, then
+// appended (an append between two loads would order them one after the other).
+__device__ __forceinline__ void push_children(const PoolView &p, uint32_t g, uint2 *front, uint32_t *count,
+                                              uint32_t cap, uint32_t *overflow) {
+  uint32_t c[8];
+#pragma unroll
+  for (uint32_t k = 0; k < 8u; k++) {
+    const uint32_t b = 8u * g + k;
+    c[k] = b < p.n_blocks ? p.blocks[b].child : kU32Max;
+  }
+#pragma unroll
+  for (uint32_t k = 0; k < 8u; k++)
+    if (c[k] != kU32Max) push(front, count, cap, overflow, c[k] >> 3, 8u * g + k);
+}
+
 // Exclusive scan of one value per thread over a work-group of WG threads; returns the
 // thread's prefix and leaves the group's total in *total (all threads).
 template <int WG>
@@ -161,6 +176,30 @@ __global__ void fill_u32_kernel(uint32_t *p, uint32_t v, size_t n) {
 }
 __global__ void fill_u64_kernel(unsigned long long *p, unsigned long long v, size_t n) {
   for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) p[i] = v;
+}
+
+// What a dispatch starts from, in one launch: cleared counters, an empty winner table, no claimed
+// groups (four launches of 3 us with gaps of 5 before).
+__global__ __launch_bounds__(kFlat) void begin_kernel(TreeScratch t) {
+  const size_t first = blockIdx.x * (size_t)kFlat + threadIdx.x, step = gridDim.x * (size_t)kFlat;
+  if (t.keys) {
+    for (size_t i = first; i <= t.table_mask; i += step) {
+      t.keys[i] = kEmptyKey;
+      t.vals[i] = 0u;
+    }
+  }
+  for (size_t i = first; i <= t.claimed_words; i += step) t.claimed[i] = 0u;
+  for (size_t i = first; i < kTcSlots; i += step) t.counters[i] = 0u;
+}
+
+// Counters to pinned host memory (the n_a words of a, then the n_b of b), then `tag` behind them: once
+// the host sees the tag the words are there.  One wave, so its fence covers every store.
+__global__ __launch_bounds__(64) void tell_kernel(const uint32_t *a, uint32_t n_a, const uint32_t *b, uint32_t n_b,
+                                                  uint32_t *host, uint32_t *host_tag, uint32_t tag) {
+  for (uint32_t i = threadIdx.x; i < n_a; i += 64u) host[i] = a[i];
+  for (uint32_t i = threadIdx.x; i < n_b; i += 64u) host[n_a + i] = b[i];
+  __threadfence_system();
+  if (threadIdx.x == 0 && host_tag) __hip_atomic_store(host_tag, tag, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // Exclusive scans over spans of kScanSpan elements.  Wave w of the work-group owns 64 *
@@ -253,9 +292,10 @@ __global__ __launch_bounds__(kScanWg) void scan_apply_kernel(const uint32_t *in,
 
 __global__ __launch_bounds__(kFlat) void prune_resolve_kernel(PoolView p, const svo_pruning *rec, uint32_t n,
                                                               uint32_t n_surface, const uint64_t *locs,
-                                                              uint32_t n_locs, ResolveOut *res, uint32_t *counters) {
+                                                              uint32_t n_locs, TreeScratch t) {
   const uint32_t i = blockIdx.x * kFlat + threadIdx.x;
   if (i >= n) return;
+  uint32_t *counters = t.counters;
   const svo_pruning r = rec[i];
   ResolveOut o{kResInvalid, 0u, 0u, 0u};
   if ((r.properties >> 4) & 1u) {
@@ -266,39 +306,49 @@ __global__ __launch_bounds__(kFlat) void prune_resolve_kernel(PoolView p, const 
   } else {
     o = resolve_target(p, r.depth, r.address, locs, n_locs);
   }
-  res[i] = o;
+  t.res[i] = o;
   if (o.status == kResMiss) counters[kTcMisses] = 1u;
   const uint32_t slot = (o.status == kResOk || o.status == kResBase) ? kTcApplied
                         : o.status == kResInvalid                   ? kTcInvalid
                                                                     : kTcSkipped;
   wave_count(counters, slot);
+  // the fields the record writes, and the group its block holds when it culls it
+  if (o.status == kResBase) win_insert(t.keys, t.vals, t.table_mask, win_key(kClsBase, o.addr), i);
+  if (o.status != kResOk) return;
+  const uint32_t a = o.addr;
+  if (r.properties & 1u) {
+    win_insert(t.keys, t.vals, t.table_mask, win_key(kClsChild, a), i);
+    if (r.child_address != kU32Max)
+      win_insert(t.keys, t.vals, t.table_mask, win_key(kClsParent, r.child_address >> 3), i);
+    const uint32_t c = p.blocks[a].child;
+    if (c != kU32Max) push(t.front[0], &counters[kTcFront0], t.front_capacity, &counters[kTcOverflow], c >> 3, a);
+  }
+  const uint32_t v = (r.properties >> 1) & 3u;
+  if ((v == 1u || v == 3u) && (a >> 3) < p.n_usages)
+    win_insert(t.keys, t.vals, t.table_mask, win_key(kClsTick, a >> 3), i);
+  if ((r.properties >> 3) & 1u) win_insert(t.keys, t.vals, t.table_mask, win_key(kClsPayload, a), i);
 }
 
+// Also enters the grafts the collected groups suffice for as writers of their targets.
 __global__ __launch_bounds__(kFlat) void graft_resolve_kernel(PoolView p, const svo_grafting *rec, uint32_t n,
-                                                              const uint32_t *need, const uint64_t *locs,
-                                                              uint32_t n_locs, ResolveOut *res, uint32_t *counters) {
+                                                              const uint64_t *locs, uint32_t n_locs,
+                                                              DevCount got_count, TreeScratch t) {
   const uint32_t i = blockIdx.x * kFlat + threadIdx.x;
   if (i >= n) return;
   ResolveOut o{kResInvalid, 0u, 0u, 0u};
-  if (need[i]) o = resolve_target(p, rec[i].depth, rec[i].graft_address, locs, n_locs);
-  res[i] = o;
-  if (o.status == kResMiss) counters[kTcMisses] = 1u;
+  const uint32_t need = t.need[i];
+  if (need) o = resolve_target(p, rec[i].depth, rec[i].graft_address, locs, n_locs);
+  t.res[i] = o;
+  if (o.status == kResMiss) t.counters[kTcMisses] = 1u;
+  if (o.status == kResOk && t.start[i] + need <= got_count.get())
+    win_insert(t.keys, t.vals, t.table_mask, win_key(kClsGraft, o.addr), i);
 }
 
-struct RecordFields {
-  const uint8_t *base;
-  uint32_t stride, depth_off, addr_off;
-  __device__ uint32_t depth(uint32_t i) const { return base[(size_t)i * stride + depth_off]; }
-  __device__ uint32_t address(uint32_t i) const {
-    return *reinterpret_cast<const uint32_t *>(base + (size_t)i * stride + addr_off);
-  }
-};
-
 // requestChild from findAddress (wavefront.cl:1201-1205): misses append in record order
-// after the current ChildRequestID; beyond capacity they are counted only.
-__global__ __launch_bounds__(kScanWg) void request_scan_kernel(PoolView p, RecordFields f, uint32_t n,
-                                                               const uint64_t *locs, const ResolveOut *res,
-                                                               uint32_t *counters) {
+// after the current ChildRequestID; beyond capacity they are counted only.  One work-group of
+// kScanWg threads.
+__device__ void request_scan(const PoolView &p, const RecordFields &f, uint32_t n, const uint64_t *locs,
+                             const ResolveOut *res, uint32_t *counters) {
   // no record missed (every graft of the streaming update addresses its block directly):
   // nothing to append, and ChildRequestID and the request count stay as they are
   if (counters[kTcMisses] == 0u) return;
@@ -360,11 +410,8 @@ __global__ __launch_bounds__(kScanWg) void request_scan_kernel(PoolView p, Recor
   }
 }
 
-__global__ __launch_bounds__(kFlat) void touch_kernel(PoolView p, RecordFields f, uint32_t n, const uint64_t *locs,
-                                                      const ResolveOut *res) {
-  const uint32_t i = blockIdx.x * kFlat + threadIdx.x;
-  if (i >= n) return;
-  const ResolveOut o = res[i];
+__device__ __forceinline__ void touch_path(const PoolView &p, const RecordFields &f, uint32_t i, const uint64_t *locs,
+                                           const ResolveOut &o) {
   if (o.status != kResOk && o.status != kResMiss) return;
   const uint32_t depth = f.depth(i);
   if (depth == 0xffu) {
@@ -375,46 +422,23 @@ __global__ __launch_bounds__(kFlat) void touch_kernel(PoolView p, RecordFields f
   }
 }
 
+// A kernel of its own: resolution tests ticks that a touch may set.
+__global__ __launch_bounds__(kFlat) void touch_kernel(PoolView p, RecordFields f, uint32_t n, const uint64_t *locs,
+                                                      const ResolveOut *res) {
+  const uint32_t i = blockIdx.x * kFlat + threadIdx.x;
+  if (i < n) touch_path(p, f, i, locs, res[i]);
+}
+
 // ---------------------------------------------------------------------------
 // prune
 // ---------------------------------------------------------------------------
 
-__global__ __launch_bounds__(kFlat) void prune_winners_kernel(PoolView p, const svo_pruning *rec, uint32_t n,
-                                                              const ResolveOut *res, unsigned long long *keys,
-                                                              uint32_t *vals, uint32_t mask) {
-  const uint32_t i = blockIdx.x * kFlat + threadIdx.x;
-  if (i >= n) return;
-  const ResolveOut o = res[i];
-  const svo_pruning r = rec[i];
-  if (o.status == kResBase) win_insert(keys, vals, mask, win_key(kClsBase, o.addr), i);
-  if (o.status != kResOk) return;
-  const uint32_t a = o.addr;
-  if (r.properties & 1u) {
-    win_insert(keys, vals, mask, win_key(kClsChild, a), i);
-    if (r.child_address != kU32Max) win_insert(keys, vals, mask, win_key(kClsParent, r.child_address >> 3), i);
-  }
-  const uint32_t v = (r.properties >> 1) & 3u;
-  if ((v == 1u || v == 3u) && (a >> 3) < p.n_usages) win_insert(keys, vals, mask, win_key(kClsTick, a >> 3), i);
-  if ((r.properties >> 3) & 1u) win_insert(keys, vals, mask, win_key(kClsPayload, a), i);
-}
-
-// CullChild roots: the group each culled block holds when the dispatch begins.
-__global__ __launch_bounds__(kFlat) void prune_roots_kernel(PoolView p, const svo_pruning *rec, uint32_t n,
-                                                            const ResolveOut *res, uint2 *front, uint32_t *counters,
-                                                            uint32_t cap) {
-  const uint32_t i = blockIdx.x * kFlat + threadIdx.x;
-  if (i >= n) return;
-  if (res[i].status != kResOk || !(rec[i].properties & 1u)) return;
-  const uint32_t a = res[i].addr;
-  const uint32_t c = p.blocks[a].child;
-  if (c != kU32Max) push(front, &counters[kTcFront0], cap, &counters[kTcOverflow], c >> 3, a);
-}
-
 __global__ __launch_bounds__(kFlat) void prune_child_kernel(PoolView p, const svo_pruning *rec, uint32_t n,
                                                             const ResolveOut *res, const unsigned long long *keys,
-                                                            const uint32_t *vals, uint32_t mask) {
+                                                            const uint32_t *vals, uint32_t mask,
+                                                            const uint32_t *counters) {
   const uint32_t i = blockIdx.x * kFlat + threadIdx.x;
-  if (i >= n) return;
+  if (i >= n || counters[kTcPending]) return;
   if (res[i].status != kResOk || !(rec[i].properties & 1u)) return;
   const uint32_t a = res[i].addr, c = rec[i].child_address;
   if (win_get(keys, vals, mask, win_key(kClsChild, a)) == i) p.blocks[a].child = c;
@@ -427,9 +451,9 @@ __global__ __launch_bounds__(kFlat) void prune_child_kernel(PoolView p, const sv
 __global__ __launch_bounds__(kFlat) void prune_fields_kernel(PoolView p, const svo_pruning *rec, uint32_t n,
                                                              const svo_block *surface, const ResolveOut *res,
                                                              const unsigned long long *keys, const uint32_t *vals,
-                                                             uint32_t mask) {
+                                                             uint32_t mask, const uint32_t *counters) {
   const uint32_t i = blockIdx.x * kFlat + threadIdx.x;
-  if (i >= n) return;
+  if (i >= n || counters[kTcPending]) return;
   const ResolveOut o = res[i];
   const svo_pruning r = rec[i];
   if (o.status == kResBase) {
@@ -472,12 +496,7 @@ __device__ void free_level(const PoolView &p, const uint2 *in, uint32_t n, uint2
       continue;
     }
     p.usages[g].tick = 0;
-    for (uint32_t k = 0; k < 8u; k++) {
-      const uint32_t b = 8u * g + k;
-      if (b >= p.n_blocks) break;
-      const uint32_t c = p.blocks[b].child;
-      if (c != kU32Max) push(out, out_count, cap, overflow, c >> 3, b);
-    }
+    push_children(p, g, out, out_count, cap, overflow);
   }
 }
 
@@ -524,8 +543,20 @@ __device__ void unlink_parent(const PoolView &p, uint32_t g, uint32_t pb) {
   }
 }
 
+// The end of a walk.  The child requests of a dispatch's missed records (n of them; 0: none) are
+// appended here, since both are one work-group's work and nothing in between reads either.  With
+// may_wait a walk that is not over is left as it stands and marked pending: the kernels after it
+// do nothing then, and the host finds the mark with its one read at the end of the dispatch, adds
+// levels and launches them again.  (Reading the frontier first cost every dispatch a stream wait
+// of 20 to 40 us, and most walks end within the first levels.)
 __global__ __launch_bounds__(kScanWg) void unlink_kernel(PoolView p, const uint2 *events, uint32_t cap,
-                                                         uint32_t levels, uint32_t *counters) {
+                                                         uint32_t levels, uint32_t may_wait, RecordFields f,
+                                                         uint32_t n_records, const uint64_t *locs,
+                                                         const ResolveOut *res, uint32_t *counters) {
+  if (n_records) request_scan(p, f, n_records, locs, res, counters);
+  const bool pending = may_wait && counters[front_slot(levels % 3u)] != 0u;
+  if (threadIdx.x == 0) counters[kTcPending] = pending ? 1u : 0u;
+  if (pending) return;
   __shared__ unsigned long long s[kUnlinkSortMax];
   const uint32_t n = counters[kTcEvents] < cap ? counters[kTcEvents] : cap;
   uint32_t m = 2;
@@ -588,33 +619,32 @@ __global__ __launch_bounds__(kFlat) void collect_count_kernel(PoolView p, uint32
                                                               uint32_t live_only, const uint32_t *claimed,
                                                               uint32_t *chunk_counts) {
   __shared__ uint32_t s_waves[kFlat / 64];
-  const uint32_t g0 = blockIdx.x * kCollectChunk + threadIdx.x * kPerThread;
+  // lanes take neighbouring groups: a count needs no order
+  const uint32_t g0 = blockIdx.x * kCollectChunk + threadIdx.x;
   uint32_t c = 0;
-  for (uint32_t j = 0; j < kPerThread; j++) c += candidate(p, g0 + j, ng, offset, claimed, live_only) ? 1u : 0u;
+#pragma unroll
+  for (uint32_t j = 0; j < kPerThread; j++)
+    c += candidate(p, g0 + j * kFlat, ng, offset, claimed, live_only) ? 1u : 0u;
   uint32_t all;
   block_scan<kFlat>(c, s_waves, &all);
   if (threadIdx.x == 0) chunk_counts[blockIdx.x] = all;
 }
 
-// k = min(candidates of this pass, need - collected), taken from list position `collected`
-__global__ void collect_limit_kernel(uint32_t *counters, DevCount need) {
-  if (threadIdx.x != 0) return;
-  const uint32_t got = counters[kTcGot], nd = need.get();
-  const uint32_t want = nd > got ? nd - got : 0u, total = counters[kTcTotal];
-  counters[kTcK] = total < want ? total : want;
-  counters[kTcFrom] = got;
-}
-
-__global__ void collect_advance_kernel(uint32_t *counters) {
-  if (threadIdx.x == 0) counters[kTcGot] += counters[kTcK];
-}
-
+// This pass takes limit = min(candidates, need - collected) groups, from list position `collected`.
+// A chunk whose first candidate lies beyond them is left unread: mostly all but a few, since a
+// graft needs thousands of groups of a pool of millions (8.4 M groups, 65,536 bricks at most: 22 -> 8 us).
 __global__ __launch_bounds__(kFlat) void collect_scatter_kernel(PoolView p, uint32_t ng, uint32_t offset,
                                                                 uint32_t live_only, const uint32_t *claimed,
-                                                                const uint32_t *chunk_offsets,
-                                                                const uint32_t *counters, uint32_t *list) {
+                                                                const uint32_t *chunk_offsets, DevCount need,
+                                                                uint32_t *counters, uint32_t *list) {
   __shared__ uint32_t s_waves[kFlat / 64];
-  const uint32_t from = counters[kTcFrom], limit = counters[kTcK];
+  const uint32_t from = counters[kTcGot], nd = need.get(), total = counters[kTcTotal];
+  const uint32_t want = nd > from ? nd - from : 0u, limit = total < want ? total : want;
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    counters[kTcK] = limit;
+    counters[kTcFrom] = from;
+  }
+  if (chunk_offsets[blockIdx.x] >= limit) return;
   const uint32_t g0 = blockIdx.x * kCollectChunk + threadIdx.x * kPerThread;
   bool is[kPerThread];
   uint32_t c = 0;
@@ -632,24 +662,20 @@ __global__ __launch_bounds__(kFlat) void collect_scatter_kernel(PoolView p, uint
 }
 
 // Claims list[from, from+k): marks them, cuts stale live groups from their parents and
-// queues what hangs below them for freeing.
+// queues what hangs below them for freeing.  The groups count as collected from here on.
 __global__ __launch_bounds__(kFlat) void collect_claim_kernel(PoolView p, const uint32_t *list, uint32_t k_max,
                                                               uint32_t *claimed, uint2 *front, uint32_t *counters,
                                                               uint32_t cap) {
   const uint32_t i = blockIdx.x * kFlat + threadIdx.x;
   const uint32_t k = counters[kTcK] < k_max ? counters[kTcK] : k_max;
+  if (i == 0) counters[kTcGot] = counters[kTcFrom] + counters[kTcK];
   if (i >= k) return;
   const uint32_t g = list[counters[kTcFrom] + i];
   atomicOr(&claimed[g >> 5], 1u << (g & 31u));
   if (p.usages[g].tick == 0) return;
   const uint32_t pb = p.usages[g].parent;
   if (pb < p.n_blocks && p.blocks[pb].child == 8u * g) p.blocks[pb].child = kU32Max;
-  for (uint32_t j = 0; j < 8u; j++) {
-    const uint32_t b = 8u * g + j;
-    if (b >= p.n_blocks) break;
-    const uint32_t c = p.blocks[b].child;
-    if (c != kU32Max) push(front, &counters[kTcFront0], cap, &counters[kTcOverflow], c >> 3, b);
-  }
+  push_children(p, g, front, &counters[kTcFront0], cap, &counters[kTcOverflow]);
 }
 
 // Claimed groups get `tick`: the frame tick when collected for a graft, 0 when reclaimed.
@@ -657,7 +683,7 @@ __global__ __launch_bounds__(kFlat) void collect_mark_kernel(PoolView p, const u
                                                              const uint32_t *counters, uint32_t tick) {
   const uint32_t i = blockIdx.x * kFlat + threadIdx.x;
   const uint32_t k = counters[kTcK] < k_max ? counters[kTcK] : k_max;
-  if (i >= k) return;
+  if (i >= k || counters[kTcPending]) return;
   const uint32_t g = list[counters[kTcFrom] + i];
   p.usages[g].tick = (uint16_t)tick;
   p.usages[g].parent = kU32Max;
@@ -675,9 +701,7 @@ __global__ __launch_bounds__(kFlat) void graft_size_kernel(const svo_grafting *r
     size[i] = 0u;  // beyond the records present: no groups, no need
     return;
   }
-  const uint32_t gda = rec[i].graft_data_address, tot = rec[i].graft_total_size;
-  const bool ok = tot >= 8u && (tot & 7u) == 0 && (gda & 7u) == 0 && (unsigned long long)gda + tot <= n_gb;
-  size[i] = ok ? tot / 8u : 0u;
+  size[i] = graft_groups(rec[i], n_gb);
 }
 
 // Pre-order numbering of each graft's groups (the depthHeap walk of wavefront.cl:1322-1349).
@@ -694,6 +718,15 @@ __global__ __launch_bounds__(64) void graft_structure_kernel(const svo_grafting 
   }
   const uint32_t gda = rec[r].graft_data_address, tot = ng * 8u;
   uint32_t *num = number + where[r], *par = parent + where[r];
+  if (ng == 1u) {  // one group, as the streaming update's bricks: valid when nothing hangs below it
+    bool leaf = true;
+#pragma unroll
+    for (uint32_t k = 0; k < 8u; k++) leaf &= gb[gda + k].child == kU32Max;
+    num[0] = 0;
+    par[0] = kU32Max;
+    need[r] = leaf ? 1u : 0u;
+    return;
+  }
   for (uint32_t q = 0; q < ng; q++) num[q] = kU32Max;
   uint32_t stack_q[64], stack_k[64];
   uint32_t top = 1, next = 1;
@@ -729,18 +762,9 @@ __global__ __launch_bounds__(64) void graft_structure_kernel(const svo_grafting 
   need[r] = (ok && next == ng) ? ng : 0u;
 }
 
-__global__ __launch_bounds__(kFlat) void graft_winners_kernel(const ResolveOut *res, const uint32_t *start,
-                                                              const uint32_t *need, uint32_t n, DevCount got_count,
-                                                              unsigned long long *keys, uint32_t *vals,
-                                                              uint32_t mask) {
-  const uint32_t i = blockIdx.x * kFlat + threadIdx.x;
-  if (i >= n) return;
-  const uint32_t got = got_count.get();
-  if (res[i].status == kResOk && start[i] + need[i] <= got) win_insert(keys, vals, mask, win_key(kClsGraft, res[i].addr), i);
-}
-
-// Decides which grafts are linked and queues what their targets held before.
-__global__ __launch_bounds__(kFlat) void graft_roots_kernel(PoolView p, ResolveOut *res, const uint32_t *start,
+// The ticks along every walk; decides which grafts are linked and queues what their targets held before.
+__global__ __launch_bounds__(kFlat) void graft_roots_kernel(PoolView p, RecordFields f, const uint64_t *locs,
+                                                            ResolveOut *res, const uint32_t *start,
                                                             const uint32_t *need, DevCount n, DevCount got_count,
                                                             const unsigned long long *keys, const uint32_t *vals,
                                                             uint32_t mask, uint2 *front, uint32_t *counters,
@@ -753,6 +777,7 @@ __global__ __launch_bounds__(kFlat) void graft_roots_kernel(PoolView p, ResolveO
   }
   const uint32_t got = got_count.get();
   const ResolveOut o = res[i];
+  touch_path(p, f, i, locs, o);
   const bool placed = o.status == kResOk && start[i] + need[i] <= got &&
                       win_get(keys, vals, mask, win_key(kClsGraft, o.addr)) == i;
   res[i].placed = placed ? 1u : 0u;
@@ -772,9 +797,10 @@ __global__ __launch_bounds__(kFlat) void graft_place_kernel(PoolView p, const sv
                                                             const ResolveOut *res, const uint32_t *start,
                                                             const uint32_t *where, const uint32_t *number,
                                                             const uint32_t *parent, const uint32_t *list, uint32_t n,
-                                                            DevCount need_count) {
+                                                            DevCount need_count, const uint32_t *counters) {
   const uint32_t t = blockIdx.x * kFlat + threadIdx.x;
   const uint32_t g = t >> 3;
+  if (counters[kTcPending]) return;
   if (g >= need_count.v || g >= need_count.get()) return;
   uint32_t lo = 0, hi = n;  // start[lo] <= g < start[hi] (start[n] taken as total_need)
   while (hi - lo > 1u) {
@@ -799,17 +825,13 @@ __global__ __launch_bounds__(kFlat) void graft_place_kernel(PoolView p, const sv
   }
 }
 
-__global__ __launch_bounds__(kFlat) void graft_link_kernel(PoolView p, const ResolveOut *res, const uint32_t *start,
-                                                           const uint32_t *list, uint32_t n) {
+// Links the placed grafts; collected groups no linked graft uses go back to the free pool.
+__global__ __launch_bounds__(kFlat) void graft_finish_kernel(PoolView p, const ResolveOut *res, const uint32_t *start,
+                                                             uint32_t n, const uint32_t *list, DevCount got,
+                                                             const uint32_t *counters) {
   const uint32_t i = blockIdx.x * kFlat + threadIdx.x;
-  if (i >= n || !res[i].placed) return;
-  p.blocks[res[i].addr].child = 8u * list[start[i]];
-}
-
-// Collected groups no linked graft uses go back to the free pool.
-__global__ __launch_bounds__(kFlat) void graft_release_kernel(PoolView p, const ResolveOut *res, const uint32_t *start,
-                                                              uint32_t n, const uint32_t *list, DevCount got) {
-  const uint32_t i = blockIdx.x * kFlat + threadIdx.x;
+  if (counters[kTcPending]) return;
+  if (i < n && res[i].placed) p.blocks[res[i].addr].child = 8u * list[start[i]];
   if (i >= got.v || i >= got.get()) return;
   // owner: the last record whose run starts at or before i
   uint32_t lo = 0, hi = n;
@@ -846,6 +868,26 @@ int tree_fill_u64(unsigned long long *p, unsigned long long value, size_t n, hip
   return launch_rc();
 }
 
+int launch_begin(const TreeScratch &t, hipStream_t s) {
+  const size_t most = std::max<size_t>(t.keys ? t.table_mask : 0u, t.claimed_words);
+  const uint32_t g = (uint32_t)std::min<size_t>(most / kFlat + 1, 1024);
+  hipLaunchKernelGGL(begin_kernel, dim3(g), dim3(kFlat), 0, s, t);
+  return launch_rc();
+}
+
+int launch_tell(const uint32_t *a, uint32_t n_a, const uint32_t *b, uint32_t n_b, uint32_t *host, uint32_t *host_tag,
+                uint32_t tag, hipStream_t s) {
+  hipLaunchKernelGGL(tell_kernel, dim3(1), dim3(64), 0, s, a, n_a, b, n_b, host, host_tag, tag);
+  return launch_rc();
+}
+
+int launch_touches(const PoolView &p, const RecordFields &f, uint32_t n, const uint64_t *locs, const TreeScratch &t,
+                   hipStream_t s) {
+  if (!n) return 0;
+  hipLaunchKernelGGL(touch_kernel, dim3(blocks_for(n)), dim3(kFlat), 0, s, p, f, n, locs, t.res);
+  return launch_rc();
+}
+
 size_t scan_span_sums_bytes(uint32_t n) {
   return n <= 2u * kScanSpan ? 0 : (size_t)(((uint64_t)n + kScanSpan - 1) / kScanSpan) * 4;
 }
@@ -874,47 +916,14 @@ int launch_prune_resolve(const PoolView &p, const svo_pruning *rec, uint32_t n, 
                          const uint64_t *locs, uint32_t n_locs, const TreeScratch &t, hipStream_t s) {
   if (!n) return 0;
   hipLaunchKernelGGL(prune_resolve_kernel, dim3(blocks_for(n)), dim3(kFlat), 0, s, p, rec, n, n_surface, locs, n_locs,
-                     t.res, t.counters);
+                     t);
   return launch_rc();
 }
 
 int launch_graft_resolve(const PoolView &p, const svo_grafting *rec, uint32_t n, const uint64_t *locs,
-                         uint32_t n_locs, const TreeScratch &t, hipStream_t s) {
+                         uint32_t n_locs, DevCount got, const TreeScratch &t, hipStream_t s) {
   if (!n) return 0;
-  hipLaunchKernelGGL(graft_resolve_kernel, dim3(blocks_for(n)), dim3(kFlat), 0, s, p, rec, n, t.need, locs, n_locs,
-                     t.res, t.counters);
-  return launch_rc();
-}
-
-int launch_requests_and_touches(const PoolView &p, const uint8_t *depths, uint32_t depth_stride,
-                                const uint32_t *addresses, uint32_t address_stride, uint32_t n,
-                                const uint64_t *locs, const TreeScratch &t, hipStream_t s) {
-  if (!n) return 0;
-  // both fields live in the same record array: express them as offsets from the depth byte
-  RecordFields f;
-  f.base = depths;
-  f.stride = depth_stride;
-  f.depth_off = 0;
-  f.addr_off = (uint32_t)(reinterpret_cast<const uint8_t *>(addresses) - depths);
-  (void)address_stride;
-  hipLaunchKernelGGL(request_scan_kernel, dim3(1), dim3(kScanWg), 0, s, p, f, n, locs, t.res, t.counters);
-  if (launch_rc()) return -1;
-  hipLaunchKernelGGL(touch_kernel, dim3(blocks_for(n)), dim3(kFlat), 0, s, p, f, n, locs, t.res);
-  return launch_rc();
-}
-
-int launch_prune_winners(const PoolView &p, const svo_pruning *rec, uint32_t n, const TreeScratch &t,
-                         hipStream_t s) {
-  if (!n) return 0;
-  hipLaunchKernelGGL(prune_winners_kernel, dim3(blocks_for(n)), dim3(kFlat), 0, s, p, rec, n, t.res, t.keys, t.vals,
-                     t.table_mask);
-  return launch_rc();
-}
-
-int launch_prune_roots(const PoolView &p, const svo_pruning *rec, uint32_t n, const TreeScratch &t, hipStream_t s) {
-  if (!n) return 0;
-  hipLaunchKernelGGL(prune_roots_kernel, dim3(blocks_for(n)), dim3(kFlat), 0, s, p, rec, n, t.res, t.front[0],
-                     t.counters, t.front_capacity);
+  hipLaunchKernelGGL(graft_resolve_kernel, dim3(blocks_for(n)), dim3(kFlat), 0, s, p, rec, n, locs, n_locs, got, t);
   return launch_rc();
 }
 
@@ -926,8 +935,10 @@ int launch_free_level(const PoolView &p, const TreeScratch &t, uint32_t level, b
   return launch_rc();
 }
 
-int launch_unlink(const PoolView &p, const TreeScratch &t, uint32_t levels, hipStream_t s) {
-  hipLaunchKernelGGL(unlink_kernel, dim3(1), dim3(kScanWg), 0, s, p, t.events, t.event_capacity, levels, t.counters);
+int launch_unlink(const PoolView &p, const TreeScratch &t, uint32_t levels, bool may_wait, const RecordFields &f,
+                  uint32_t n_records, const uint64_t *locs, hipStream_t s) {
+  hipLaunchKernelGGL(unlink_kernel, dim3(1), dim3(kScanWg), 0, s, p, t.events, t.event_capacity, levels,
+                     may_wait ? 1u : 0u, f, n_records, locs, t.res, t.counters);
   return launch_rc();
 }
 
@@ -935,10 +946,10 @@ int launch_prune_apply(const PoolView &p, const svo_pruning *rec, uint32_t n, co
                        const TreeScratch &t, hipStream_t s) {
   if (!n) return 0;
   hipLaunchKernelGGL(prune_child_kernel, dim3(blocks_for(n)), dim3(kFlat), 0, s, p, rec, n, t.res, t.keys, t.vals,
-                     t.table_mask);
+                     t.table_mask, t.counters);
   if (launch_rc()) return -1;
   hipLaunchKernelGGL(prune_fields_kernel, dim3(blocks_for(n)), dim3(kFlat), 0, s, p, rec, n, surface, t.res, t.keys,
-                     t.vals, t.table_mask);
+                     t.vals, t.table_mask, t.counters);
   return launch_rc();
 }
 
@@ -952,22 +963,12 @@ int launch_collect_count(const PoolView &p, uint32_t n_groups, uint32_t offset, 
   return launch_scan_u32(t.chunk_counts, t.chunk_counts, chunks, &t.counters[kTcTotal], t.scan_sums, s);
 }
 
-int launch_collect_limit(const TreeScratch &t, DevCount need, hipStream_t s) {
-  hipLaunchKernelGGL(collect_limit_kernel, dim3(1), dim3(64), 0, s, t.counters, need);
-  return launch_rc();
-}
-
-int launch_collect_advance(const TreeScratch &t, hipStream_t s) {
-  hipLaunchKernelGGL(collect_advance_kernel, dim3(1), dim3(64), 0, s, t.counters);
-  return launch_rc();
-}
-
-int launch_collect_scatter(const PoolView &p, uint32_t n_groups, uint32_t offset, bool live_only,
+int launch_collect_scatter(const PoolView &p, uint32_t n_groups, uint32_t offset, bool live_only, DevCount need,
                            const TreeScratch &t, hipStream_t s) {
   const uint32_t chunks = (n_groups + kCollectChunk - 1u) / kCollectChunk;
   if (!chunks) return 0;
   hipLaunchKernelGGL(collect_scatter_kernel, dim3(chunks), dim3(kFlat), 0, s, p, n_groups, offset,
-                     live_only ? 1u : 0u, t.claimed, t.chunk_counts, t.counters, t.list);
+                     live_only ? 1u : 0u, t.claimed, t.chunk_counts, need, t.counters, t.list);
   return launch_rc();
 }
 
@@ -1000,18 +1001,11 @@ int launch_graft_sizes(const svo_grafting *rec, DevCount n, uint32_t n_gb, const
   return launch_rc();
 }
 
-int launch_graft_winners(const PoolView &p, uint32_t n, DevCount got, const TreeScratch &t, hipStream_t s) {
-  (void)p;
-  if (!n) return 0;
-  hipLaunchKernelGGL(graft_winners_kernel, dim3(blocks_for(n)), dim3(kFlat), 0, s, t.res, t.start, t.need, n, got,
-                     t.keys, t.vals, t.table_mask);
-  return launch_rc();
-}
-
-int launch_graft_roots(const PoolView &p, DevCount n, DevCount got, const TreeScratch &t, hipStream_t s) {
+int launch_graft_roots(const PoolView &p, const RecordFields &f, DevCount n, const uint64_t *locs, DevCount got,
+                       const TreeScratch &t, hipStream_t s) {
   if (!n.v) return 0;
-  hipLaunchKernelGGL(graft_roots_kernel, dim3(blocks_for(n.v)), dim3(kFlat), 0, s, p, t.res, t.start, t.need, n, got,
-                     t.keys, t.vals, t.table_mask, t.front[0], t.counters, t.front_capacity);
+  hipLaunchKernelGGL(graft_roots_kernel, dim3(blocks_for(n.v)), dim3(kFlat), 0, s, p, f, locs, t.res, t.start, t.need, n,
+                     got, t.keys, t.vals, t.table_mask, t.front[0], t.counters, t.front_capacity);
   return launch_rc();
 }
 
@@ -1021,17 +1015,16 @@ int launch_graft_place(const PoolView &p, const svo_grafting *rec, uint32_t n, D
   if (total_need.v) {
     const uint32_t blocks = (uint32_t)((8ull * total_need.v + kFlat - 1) / kFlat);
     hipLaunchKernelGGL(graft_place_kernel, dim3(blocks), dim3(kFlat), 0, s, p, rec, gb, t.res, t.start, t.where,
-                       t.number, t.parent, t.list, n, total_need);
+                       t.number, t.parent, t.list, n, total_need, t.counters);
   }
-  if (launch_rc()) return -1;
-  hipLaunchKernelGGL(graft_link_kernel, dim3(blocks_for(n)), dim3(kFlat), 0, s, p, t.res, t.start, t.list, n);
   return launch_rc();
 }
 
-int launch_graft_release(const PoolView &p, uint32_t n, DevCount got, const TreeScratch &t, hipStream_t s) {
-  if (!got.v) return 0;
-  hipLaunchKernelGGL(graft_release_kernel, dim3(blocks_for(got.v)), dim3(kFlat), 0, s, p, t.res, t.start, n, t.list,
-                     got);
+int launch_graft_finish(const PoolView &p, uint32_t n, DevCount got, const TreeScratch &t, hipStream_t s) {
+  const uint32_t most = std::max(n, got.v);
+  if (!most) return 0;
+  hipLaunchKernelGGL(graft_finish_kernel, dim3(blocks_for(most)), dim3(kFlat), 0, s, p, t.res, t.start, n, t.list, got,
+                     t.counters);
   return launch_rc();
 }
 
