@@ -418,13 +418,13 @@ extern "C" int svo_stream_update(svo_context *ctx, const svo_terrain *t, const s
     uint32_t *flags = (uint32_t *)p;
     if ((rc = st.grow(kSbList, (size_t)std::max(1u, std::min(stored, max_bricks)) * 4, &p))) return rc;
     uint32_t *list = (uint32_t *)p;
-    if ((rc = st.launch(launch_request_unique(src, stored, state + kShStored,
-                                              first, ctx->stream_gen, (const uint4 *)pv.blocks, pv.n_blocks,
-                                              o->max_depth, flags, s),
-                        "request unique")))
-      return rc;
     const uint32_t chunks = (stored + 1023u) / 1024u;
     if ((rc = st.grow(kSbCounts, ((size_t)chunks + kShSlots) * 4, &p))) return rc;
+    if ((rc = st.launch(launch_request_unique(src, stored, state + kShStored,
+                                              first, ctx->stream_gen, (const uint4 *)pv.blocks, pv.n_blocks,
+                                              o->max_depth, flags, (uint32_t *)p, s),
+                        "request unique")))
+      return rc;
     uint32_t *sums = nullptr;
     if ((rc = context_scan_sums(ctx, scan_span_sums_bytes(chunks), &sums))) return rc;
     if ((rc = st.launch(launch_rank(flags, stored, (uint32_t *)p, nullptr, state + kShUnique, sums, s, list,

@@ -44,10 +44,11 @@ struct RequestSource {
 };
 // flags[i] (i < min(*n, n_max), not written beyond) = 1 for the first request of each block
 // that can take a child level among the *n stored requests; first: u64 per block of the
-// pool, entries of generations below gen are ignored (zero-filled when allocated)
+// pool, entries of generations below gen are ignored (zero-filled when allocated); counts[c] =
+// flags of requests [1024 c, 1024 (c + 1)), for every chunk of n_max
 int launch_request_unique(const RequestSource &req, uint32_t n_max, const uint32_t *n, unsigned long long *first,
                           uint32_t gen, const uint4 *blocks, uint32_t n_blocks, uint32_t max_depth, uint32_t *flags,
-                          hipStream_t s);
+                          uint32_t *counts, hipStream_t s);
 // bricks of the first min(*unique, nb_max) listed requests
 int launch_bricks(const TerrainView &t, const RequestSource &req, const uint32_t *list, uint32_t nb_max,
                   const uint32_t *unique, svo_grafting *records, uint4 *bricks, hipStream_t s);

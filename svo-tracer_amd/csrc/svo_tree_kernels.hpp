@@ -166,9 +166,11 @@ int launch_collect_claim(const PoolView &p, uint32_t k_max, const TreeScratch &t
 int launch_collect_mark(const PoolView &p, uint32_t k_max, uint32_t tick, const TreeScratch &t, hipStream_t s);
 
 // graft
-// n.v records are processed; those at or beyond n.get() count as absent (size and need 0)
-int launch_graft_sizes(const svo_grafting *rec, DevCount n, uint32_t n_gb, const TreeScratch &t, hipStream_t s);
-int launch_graft_structure(const svo_grafting *rec, uint32_t n, const svo_block *gb, uint32_t n_gb,
+int launch_graft_sizes(const svo_grafting *rec, uint32_t n, uint32_t n_gb, const TreeScratch &t, hipStream_t s);
+// n.v records are processed.  Host-known count: sizes and their scan (t.size, t.where) are there.
+// Device count: records at or beyond it count as absent (need 0), and no two grafts share graft
+// blocks, so each graft's numbering starts at its first block's group (t.where is set here).
+int launch_graft_structure(const svo_grafting *rec, DevCount n, const svo_block *gb, uint32_t n_gb,
                            const TreeScratch &t, hipStream_t s);
 // Exclusive scan of n u32; the sum goes to *total.  Above 2 x 16384 elements the scan needs
 // span_sums, device scratch of scan_span_sums_bytes(n) bytes owned by the caller.

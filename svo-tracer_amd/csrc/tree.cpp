@@ -350,28 +350,29 @@ int graft_impl(Context *ctx, const Pool &pool, const svo_update_input_data &in, 
   op.ts.start = (uint32_t *)p;
   if ((rc = op.begin())) return rc;
   const DevCount records{n, dev_records};
-  // structure: sizes, where each graft's numbering lives, pre-order numbering, needs
-  if ((rc = op.launch(launch_graft_sizes(rec, records, n_gb, op.ts, s), "graft sizes"))) return rc;
+  // structure: sizes, where each graft's numbering lives, pre-order numbering, needs.  Groups of
+  // all grafts: added up here for records the host has, read back for bound ones; for counted
+  // ones every graft's groups lie in its own part of the graft blocks, so n_gb / 8 bounds them
   uint32_t *sums = nullptr;
   if ((rc = context_scan_sums(ctx, scan_span_sums_bytes(n), &sums))) return rc;
-  if ((rc = op.launch(launch_scan_u32(op.ts.size, op.ts.where, n, op.ts.counters + kTcTotal, sums, s), "scan")))
-    return rc;
-  // groups of all grafts: added up here for records the host has, read back for bound ones; for
-  // counted ones every graft's groups lie in its own part of the graft blocks, so n_gb / 8
-  // bounds them
   uint32_t groups = n_gb / 8u;
-  if (host_records) {
-    groups = 0;
-    for (uint32_t i = 0; i < n; i++) groups += graft_groups(host_records[i], n_gb);
-  } else if (!dev_records) {
-    if ((rc = op.peek())) return rc;
-    groups = op.host[kTcTotal];
+  if (!dev_records) {
+    if ((rc = op.launch(launch_graft_sizes(rec, n, n_gb, op.ts, s), "graft sizes"))) return rc;
+    if ((rc = op.launch(launch_scan_u32(op.ts.size, op.ts.where, n, op.ts.counters + kTcTotal, sums, s), "scan")))
+      return rc;
+    if (host_records) {
+      groups = 0;
+      for (uint32_t i = 0; i < n; i++) groups += graft_groups(host_records[i], n_gb);
+    } else {
+      if ((rc = op.peek())) return rc;
+      groups = op.host[kTcTotal];
+    }
   }
   if ((rc = op.grow(kTbNumber, ((size_t)groups + 1) * 4, &p))) return rc;
   op.ts.number = (uint32_t *)p;
   if ((rc = op.grow(kTbParent, ((size_t)groups + 1) * 4, &p))) return rc;
   op.ts.parent = (uint32_t *)p;
-  if ((rc = op.launch(launch_graft_structure(rec, n, gb, n_gb, op.ts, s), "graft structure"))) return rc;
+  if ((rc = op.launch(launch_graft_structure(rec, records, gb, n_gb, op.ts, s), "graft structure"))) return rc;
   if ((rc = op.launch(launch_scan_u32(op.ts.need, op.ts.start, n, op.ts.counters + kTcNeed, sums, s), "scan")))
     return rc;
   // every need is at most its graft's size, so `groups` bounds the total need

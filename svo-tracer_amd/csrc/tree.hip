@@ -693,30 +693,29 @@ __global__ __launch_bounds__(kFlat) void collect_mark_kernel(PoolView p, const u
 // graft (wavefront.cl:1306-1350, as intended)
 // ---------------------------------------------------------------------------
 
-__global__ __launch_bounds__(kFlat) void graft_size_kernel(const svo_grafting *rec, DevCount n, uint32_t n_gb,
+__global__ __launch_bounds__(kFlat) void graft_size_kernel(const svo_grafting *rec, uint32_t n, uint32_t n_gb,
                                                            uint32_t *size) {
   const uint32_t i = blockIdx.x * kFlat + threadIdx.x;
-  if (i >= n.v) return;
-  if (i >= n.get()) {
-    size[i] = 0u;  // beyond the records present: no groups, no need
-    return;
-  }
-  size[i] = graft_groups(rec[i], n_gb);
+  if (i < n) size[i] = graft_groups(rec[i], n_gb);
 }
 
 // Pre-order numbering of each graft's groups (the depthHeap walk of wavefront.cl:1322-1349).
-__global__ __launch_bounds__(64) void graft_structure_kernel(const svo_grafting *rec, uint32_t n,
+// With counted records, whose groups lie each in their own part of the n_gb graft blocks, a graft's
+// numbering lies where its blocks do: no sizes to scan (five launches of a 65,536-brick update).
+__global__ __launch_bounds__(64) void graft_structure_kernel(const svo_grafting *rec, DevCount n, uint32_t n_gb,
                                                              const svo_block *gb, const uint32_t *size,
-                                                             const uint32_t *where, uint32_t *number,
-                                                             uint32_t *parent, uint32_t *need) {
+                                                             uint32_t *where, uint32_t *number, uint32_t *parent,
+                                                             uint32_t *need) {
   const uint32_t r = blockIdx.x * 64u + threadIdx.x;
-  if (r >= n) return;
-  const uint32_t ng = size[r];
-  if (!ng) {
+  if (r >= n.v) return;
+  const uint32_t ng = !n.p ? size[r] : r < n.get() ? graft_groups(rec[r], n_gb) : 0u;
+  if (!ng) {  // beyond the records present, or not whole groups of the graft blocks
+    if (n.p) where[r] = 0;
     need[r] = 0;
     return;
   }
   const uint32_t gda = rec[r].graft_data_address, tot = ng * 8u;
+  if (n.p) where[r] = gda / 8u;
   uint32_t *num = number + where[r], *par = parent + where[r];
   if (ng == 1u) {  // one group, as the streaming update's bricks: valid when nothing hangs below it
     bool leaf = true;
@@ -986,18 +985,17 @@ int launch_collect_mark(const PoolView &p, uint32_t k_max, uint32_t tick, const 
   return launch_rc();
 }
 
-int launch_graft_structure(const svo_grafting *rec, uint32_t n, const svo_block *gb, uint32_t n_gb,
+int launch_graft_structure(const svo_grafting *rec, DevCount n, const svo_block *gb, uint32_t n_gb,
                            const TreeScratch &t, hipStream_t s) {
-  (void)n_gb;
-  if (!n) return 0;
-  hipLaunchKernelGGL(graft_structure_kernel, dim3((n + 63u) / 64u), dim3(64), 0, s, rec, n, gb, t.size, t.where,
-                     t.number, t.parent, t.need);
+  if (!n.v) return 0;
+  hipLaunchKernelGGL(graft_structure_kernel, dim3((n.v + 63u) / 64u), dim3(64), 0, s, rec, n, n_gb, gb, t.size,
+                     t.where, t.number, t.parent, t.need);
   return launch_rc();
 }
 
-int launch_graft_sizes(const svo_grafting *rec, DevCount n, uint32_t n_gb, const TreeScratch &t, hipStream_t s) {
-  if (!n.v) return 0;
-  hipLaunchKernelGGL(graft_size_kernel, dim3(blocks_for(n.v)), dim3(kFlat), 0, s, rec, n, n_gb, t.size);
+int launch_graft_sizes(const svo_grafting *rec, uint32_t n, uint32_t n_gb, const TreeScratch &t, hipStream_t s) {
+  if (!n) return 0;
+  hipLaunchKernelGGL(graft_size_kernel, dim3(blocks_for(n)), dim3(kFlat), 0, s, rec, n, n_gb, t.size);
   return launch_rc();
 }
 
