@@ -6,7 +6,7 @@
 // pass, once for the groups of grafts whose records it has not seen, and again for a free walk
 // that has not ended within its first kSpecLevels levels (each level reads its frontier size on
 // the device; what follows the walk is launched with it and does nothing while it is not over).
-// A prune and a graft of 4096 records: 52 launches, 6 uploads and 6 waits -> 27 launches and 3
+// A prune and a graft of 4096 records: 52 launches, 6 uploads and 6 waits -> 34 launches and 3
 // waits.
 #include <hip/hip_runtime.h>
 
