@@ -34,6 +34,9 @@ DeviceBuffer::~DeviceBuffer() {
 }
 
 int hip_fail(hipError_t e, const char *what) {
+  // Reported here, so no longer the thread's last error: HIP keeps it through later successful calls,
+  // and the next launch, which asks for it, would fail in its place.
+  (void)hipGetLastError();
   return fail(e == hipErrorOutOfMemory ? SVO_ERR_OUT_OF_MEMORY : SVO_ERR_HIP,
               std::string(what) + ": " + hipGetErrorString(e));
 }
