@@ -261,7 +261,8 @@ int svo_zero_id(svo_context *ctx, int buffer_name);
 /* Swap, ComputeManager.cs:251-256: exchanges the handles; kernel arguments bound to either
  * name must be re-bound afterwards, as in the reference. */
 int svo_swap(svo_context *ctx, int buffer_a, int buffer_b);
-/* Device address of a named buffer (for zero-copy interop; valid until re-init/release). */
+/* Device address of a named buffer (for zero-copy interop; valid until re-init/release, and for
+ * Bases, Blocks and Usages until the next device build). */
 int svo_buffer_device_pointer(svo_context *ctx, int buffer_name, void **device_ptr);
 
 /* ---- kernels: SetArg / Enqueue / Wait / Flush, ComputeManager.cs:72-120, 277-281 ---- */
@@ -587,7 +588,12 @@ int svo_terrain_heights(const svo_terrain *terrain, float *dst, size_t count);
  * Bases and Blocks (and Usages, as svo_context_load_tree sets them, when with_usages);
  * *out (optional) receives a host copy, *block_count (optional) the block count.  As there,
  * a free-group queue that runs out at a dense-level block is SVO_ERR_CAPACITY, and one that
- * runs out deeper leaves the remaining blocks childless.  base_depth 1..7, max_depth <= 20. */
+ * runs out deeper leaves the remaining blocks childless.  base_depth 1..7, max_depth <= 20.
+ * Blocks (and Usages) of about the same size that only the context holds -- no kernel argument
+ * is bound to them -- are written over, once the device is idle; otherwise new buffers take
+ * the names.  A device pointer to them from before the build then shows the new tree.  A build
+ * that fails leaves the last tree as it was, or, when it had begun to write over it, Bases,
+ * Blocks and Usages uninitialised. */
 int svo_terrain_build_tree(svo_context *ctx, const svo_terrain *terrain, uint32_t base_depth, uint32_t max_depth,
                            uint32_t max_size, int with_usages, uint16_t usage_tick, svo_tree **out,
                            uint32_t *block_count);

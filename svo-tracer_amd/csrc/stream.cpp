@@ -601,6 +601,17 @@ struct Builder {
 
 namespace {
 
+// A build over the last tree's buffers that does not finish leaves neither tree, so it takes all three
+// names away: frames are then refused, instead of walking old Bases into new Blocks.
+struct Overwritten {
+  Context *ctx;
+  bool on = false;
+  ~Overwritten() {
+    if (!on) return;
+    for (int name : {SVO_BUF_BASES, SVO_BUF_BLOCKS, SVO_BUF_USAGES}) ctx->buffers.erase(name);
+  }
+};
+
 int build_tree_device(Context *ctx, const GeomView &g, uint32_t base_depth, uint32_t max_depth, uint32_t max_size,
                       int with_usages, uint16_t usage_tick, svo_tree **out, uint32_t *block_count) {
   Builder bd(ctx);
@@ -732,8 +743,9 @@ int build_tree_device(Context *ctx, const GeomView &g, uint32_t base_depth, uint
   const uint64_t groups64 = dense_groups + (taken > n_empties ? taken - n_empties : 0);
   if (groups64 * 8 > 0xffffffffull) return fail(SVO_ERR_CAPACITY, "svo_terrain_build_tree: more than 2^32 blocks");
   const uint32_t n_groups = (uint32_t)groups64;
-  // Everything that can be refused has been.  A tree of about the last one's size is written over
-  // it, after whatever still reads that (as freeing it would wait).
+  // Everything that can be refused is refused by the end of these allocations.  A tree of about the
+  // last one's size is written over it, after whatever still reads that (as freeing it would wait);
+  // after that only a call that fails outright ends the build.
   std::shared_ptr<DeviceBuffer> blocks, usages;
   Piece post, gparent;
   bool in_place = false;
@@ -743,6 +755,7 @@ int build_tree_device(Context *ctx, const GeomView &g, uint32_t base_depth, uint
     return rc;
   if (in_place && hipDeviceSynchronize() != hipSuccess)
     return hip_fail(hipGetLastError(), "svo_terrain_build_tree: sync");
+  Overwritten overwritten{ctx, in_place};
   // only the dense groups can stay unwritten: every other group in use is a FIFO entry that was
   // taken, with a parent and eight blocks
   if ((rc = bd.fill(blocks->ptr, 0, (size_t)dense_groups * 128)) ||
@@ -851,6 +864,7 @@ int build_tree_device(Context *ctx, const GeomView &g, uint32_t base_depth, uint
   ctx->buffers[SVO_BUF_BASES] = bases_out;
   ctx->buffers[SVO_BUF_BLOCKS] = blocks;
   if (usages) ctx->buffers[SVO_BUF_USAGES] = usages;
+  overwritten.on = false;
   bd.keep();
   ctx->tree_max_depth = max_depth;
   return SVO_OK;
