@@ -241,7 +241,8 @@ int svo_abi_version(void);
  * Re-initialising a name releases the old allocation, as the reference does.
  * host_data may be NULL (device-only buffer, zero-filled). */
 int svo_buffer_init(svo_context *ctx, int buffer_name, size_t bytes, const void *host_data, uint32_t flags);
-/* Release one named buffer (part of Dispose, ComputeManager.cs:359-360). */
+/* Release one named buffer (part of Dispose, ComputeManager.cs:359-360).  Releasing Blocks also
+ * frees what a device build kept for the next one. */
 int svo_buffer_release(svo_context *ctx, int buffer_name);
 int svo_buffer_size(svo_context *ctx, int buffer_name, size_t *bytes);
 /* WriteBuffer<T>, ComputeManager.cs:217-223 (the copy is complete when the call returns). */
@@ -593,7 +594,9 @@ int svo_terrain_heights(const svo_terrain *terrain, float *dst, size_t count);
  * is bound to them -- are written over, once the device is idle; otherwise new buffers take
  * the names.  A device pointer to them from before the build then shows the new tree.  A build
  * that fails leaves the last tree as it was, or, when it had begun to write over it, Bases,
- * Blocks and Usages uninitialised. */
+ * Blocks and Usages uninitialised.  The context keeps up to 512 MiB of the build's temporary
+ * device memory for the next one; it is freed when Blocks is released, when the context is
+ * destroyed, and when any allocation of the library on the device would fail otherwise. */
 int svo_terrain_build_tree(svo_context *ctx, const svo_terrain *terrain, uint32_t base_depth, uint32_t max_depth,
                            uint32_t max_size, int with_usages, uint16_t usage_tick, svo_tree **out,
                            uint32_t *block_count);

@@ -10,8 +10,10 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <iterator>
 #include <map>
 #include <memory>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -41,11 +43,60 @@ int hip_fail(hipError_t e, const char *what) {
               std::string(what) + ": " + hipGetErrorString(e));
 }
 
+namespace {
+
+using Buffers = std::vector<std::shared_ptr<DeviceBuffer>>;
+
+struct Kept {
+  std::mutex mutex;
+  std::map<const Context *, Buffers> of;
+};
+
+Kept &kept() {
+  static Kept *k = new Kept;  // never destroyed: the HIP runtime may be gone first
+  return *k;
+}
+
+// Frees what the current device's contexts keep; false when there is nothing.
+bool give_back() {
+  int device = 0;
+  if (hipGetDevice(&device) != hipSuccess) return false;
+  Buffers freed;  // outside the lock: a free waits for the device
+  std::lock_guard<std::mutex> lock(kept().mutex);
+  for (auto &k : kept().of) {
+    if (k.first->device != device) continue;
+    std::move(k.second.begin(), k.second.end(), std::back_inserter(freed));
+    k.second.clear();
+  }
+  return !freed.empty();
+}
+
+}  // namespace
+
+void keep(const Context *ctx, Buffers buffers) {
+  std::lock_guard<std::mutex> lock(kept().mutex);
+  kept().of[ctx].swap(buffers);
+}
+
+Buffers take_kept(const Context *ctx) {
+  Buffers own;
+  std::lock_guard<std::mutex> lock(kept().mutex);
+  auto it = kept().of.find(ctx);
+  if (it == kept().of.end()) return own;
+  own.swap(it->second);
+  kept().of.erase(it);
+  return own;
+}
+
 int new_buffer(size_t bytes, std::shared_ptr<DeviceBuffer> *out) {
   auto b = std::make_shared<DeviceBuffer>();
   b->bytes = b->capacity = bytes;
   if (bytes) {
     hipError_t e = hipMalloc(&b->ptr, bytes);
+    if (e == hipErrorOutOfMemory && give_back()) {
+      (void)hipGetLastError();
+      e = hipMalloc(&b->ptr, bytes);
+    }
     if (e != hipSuccess) return hip_fail(e, "hipMalloc");
   }
   *out = b;
@@ -181,6 +232,7 @@ int svo_destroy(svo_context *ctx) {
   (void)hipEventDestroy(ctx->timer_begin);
   (void)hipEventDestroy(ctx->timer_end);
   for (auto &b : ctx->tree_scratch) b.reset();
+  (void)take_kept(ctx);
   if (ctx->tree_host) (void)hipHostFree(ctx->tree_host);
   if (ctx->stream_host) (void)hipHostFree(ctx->stream_host);
   if (ctx->id_host) (void)hipHostFree(ctx->id_host);
@@ -218,6 +270,7 @@ int svo_buffer_release(svo_context *ctx, int name) {
   if (it == ctx->buffers.end()) return fail(SVO_ERR_UNKNOWN_BUFFER, "svo_buffer_release: buffer not initialised");
   HIP_TRY(hipStreamSynchronize(ctx->stream), "svo_buffer_release: sync");
   ctx->buffers.erase(it);
+  if (name == SVO_BUF_BLOCKS) (void)take_kept(ctx);  // the scene goes, and what its build left with it
   return SVO_OK;
 }
 

@@ -502,7 +502,7 @@ struct BuildLevel {
 // 256 MiB) or what the piece needs.  Some fifty allocations and as many frees of a depth-12 build
 // (70 and 180 us each, and many milliseconds each when the driver has to give memory back first)
 // took longer than its kernels, so a build that succeeds leaves up to kKeptBuildBytes of its slabs
-// to the context for the next one.
+// to the context for the next one (until Blocks is released or an allocation needs the room).
 constexpr size_t kKeptBuildBytes = (size_t)512 << 20;
 
 struct Builder {
@@ -511,7 +511,7 @@ struct Builder {
   std::vector<std::shared_ptr<DeviceBuffer>> slabs, kept;
   size_t used = 0, next = (size_t)32 << 20;
 
-  explicit Builder(Context *c) : ctx(c), s(c->stream), kept(std::move(c->build_slabs)) { c->build_slabs.clear(); }
+  explicit Builder(Context *c) : ctx(c), s(c->stream), kept(take_kept(c)) {}
 
   int buf(size_t bytes, Piece *out) {
     bytes = (std::max<size_t>(bytes, 4) + 255) & ~(size_t)255;
@@ -541,16 +541,17 @@ struct Builder {
     used += bytes;
     return SVO_OK;
   }
-  // Leaves the slabs to the context (the stream orders the next build's use of them after this
-  // one's).
+  // Leaves the slabs to the context, once the build's last use of them is over.
   void keep() {
+    std::vector<std::shared_ptr<DeviceBuffer>> left;
     size_t total = 0;
     for (auto *from : {&slabs, &kept})
       for (auto &b : *from)
         if (total + b->bytes <= kKeptBuildBytes) {
           total += b->bytes;
-          ctx->build_slabs.push_back(b);
+          left.push_back(b);
         }
+    svo::keep(ctx, std::move(left));
   }
   // A named buffer of `bytes`: the context's own when nothing else holds it and it fits (and is no
   // more than twice as large), a new one otherwise.  *in_place: the caller's other streams may

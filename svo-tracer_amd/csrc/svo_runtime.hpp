@@ -39,6 +39,12 @@ int hip_fail(hipError_t e, const char *what);
 int new_buffer(size_t bytes, std::shared_ptr<DeviceBuffer> *out);
 int ensure_scratch(std::shared_ptr<DeviceBuffer> &b, size_t bytes);
 struct Context;
+// Idle device memory that contexts keep for their next device build.  It is the contexts' only until
+// an allocation on the device does not fit: new_buffer then frees what every context of the device
+// keeps and tries again.  take_kept hands a context its own back; keep and take may be called from
+// several threads.
+void keep(const Context *ctx, std::vector<std::shared_ptr<DeviceBuffer>> buffers);
+std::vector<std::shared_ptr<DeviceBuffer>> take_kept(const Context *ctx);
 // The context's span-sum scratch, grown to `bytes` (null when bytes is 0).
 int context_scan_sums(Context *ctx, size_t bytes, uint32_t **out);
 const std::vector<std::string> &kernel_params(int kernel);
@@ -159,8 +165,6 @@ struct Context {
   } kept;
   // span sums of the multi-work-group scans (tree management, streaming, device builds)
   std::shared_ptr<DeviceBuffer> scan_sums;
-  // temporaries of the last device build, kept for the next one (at most kKeptBuildBytes)
-  std::vector<std::shared_ptr<DeviceBuffer>> build_slabs;
   unsigned long long *id_host = nullptr;  // pinned word of the queue-counter read-backs (svo_reset_id)
   uint32_t id_tag = 0;                    // the last read-back's number
   // batched cameras: concatenated camera tables (cache key), camera records

@@ -8,14 +8,17 @@
 #include <cstdlib>
 #include <cstring>
 #include <map>
+#include <mutex>
 #include <string>
 #include <vector>
 
 namespace {
 
+std::mutex g_mutex;  // the calls come from several threads
+using Lock = std::lock_guard<std::mutex>;
 std::map<const void *, size_t> g_live;
 size_t g_used = 0, g_limit = (size_t)4 << 30;
-hipError_t g_last = hipSuccess;
+thread_local hipError_t g_last = hipSuccess;
 std::string g_fail_call;
 int g_fail_after = -1;
 std::map<const void *, std::string> g_names;
@@ -24,7 +27,8 @@ struct Config {
   dim3 grid, block;
   size_t shared;
   hipStream_t stream;
-} g_config;
+};
+thread_local Config g_config;
 
 hipError_t result(hipError_t e) {
   if (e != hipSuccess) g_last = e;
@@ -32,7 +36,10 @@ hipError_t result(hipError_t e) {
 }
 // Whether this call is the one to fail.
 bool fails(const char *call) { return g_fail_after >= 0 && g_fail_call == call && g_fail_after-- == 0; }
-hipError_t step(const char *call) { return result(fails(call) ? hipErrorUnknown : hipSuccess); }
+hipError_t step(const char *call) {
+  Lock lock(g_mutex);
+  return result(fails(call) ? hipErrorUnknown : hipSuccess);
+}
 
 }  // namespace
 
@@ -51,6 +58,7 @@ size_t fake_launches() { return g_launches.size(); }
 
 // ---- memory ----
 hipError_t hipMalloc(void **p, size_t bytes) {
+  Lock lock(g_mutex);
   *p = nullptr;
   if (fails("hipMalloc") || bytes > g_limit || g_used > g_limit - bytes) return result(hipErrorOutOfMemory);
   *p = std::calloc(1, bytes);
@@ -60,6 +68,7 @@ hipError_t hipMalloc(void **p, size_t bytes) {
   return hipSuccess;
 }
 hipError_t hipFree(void *p) {
+  Lock lock(g_mutex);
   auto it = g_live.find(p);
   if (it == g_live.end()) return result(hipErrorInvalidValue);
   g_used -= it->second;
@@ -111,7 +120,10 @@ hipError_t __hipPopCallConfiguration(dim3 *grid, dim3 *block, size_t *shared, hi
   return hipSuccess;
 }
 hipError_t hipLaunchKernel(const void *f, dim3, dim3, void **, size_t, hipStream_t) {
-  g_launches.push_back(g_names[f]);
+  {
+    Lock lock(g_mutex);
+    g_launches.push_back(g_names[f]);
+  }
   return step("hipLaunchKernel");
 }
 hipError_t hipOccupancyMaxActiveBlocksPerMultiprocessor(int *n, const void *, int block, size_t) {

@@ -3,6 +3,8 @@ error until it is asked for, and the launches ask, so a failure that was already
 good by a smaller allocation) must not fail the next call."""
 from __future__ import annotations
 
+import textwrap
+
 import numpy as np
 import pytest
 
@@ -34,6 +36,65 @@ def test_build_falls_back_to_what_it_needs(fake):
         cm.BuildTreeDevice(geometry, 1, 4)
         assert fake.fake_launches() > 5
     """)
+
+
+KEPT = """
+    import threading
+    geometry = svo.scenes.sphere_noise_scene(seed=1, max_depth=4, base_depth=1).geometry
+    before = fake.fake_used()
+    cm.BuildTreeDevice(geometry, 1, 4)
+    kept = fake.fake_used() - before
+    assert kept > 16 * MiB  # a build's temporaries stay for the next one
+"""
+
+
+@pytest.mark.parametrize("code", [
+    """
+    fake.fake_limit(fake.fake_used() + 8 * MiB)
+    cm.InitDeviceBuffer(B.OutputImage, kept // 2, 1)  # a buffer of the same context
+    assert fake.fake_used() < before + kept
+    """, """
+    other = svo.ComputeManager(0)
+    fake.fake_limit(fake.fake_used() + 8 * MiB)
+    other.InitDeviceBuffer(B.OutputImage, kept // 2, 1)  # of another one on the device
+    cm.BuildTreeDevice(geometry, 1, 4)  # finds nothing kept
+    """, """
+    fake.fake_limit(fake.fake_used() + 8 * MiB)
+    try:
+        cm.InitDeviceBuffer(B.OutputImage, 64 * MiB, 1)  # does not fit without them either
+        raise SystemExit("an allocation beyond the device was accepted")
+    except svo.SvoError as e:
+        assert "out of memory" in str(e), e
+    """, """
+    cm.ReleaseBuffer(B.Blocks)  # the scene goes, and what its build left with it
+    assert fake.fake_used() < before + MiB
+    """, """
+    cm.Dispose()
+    assert fake.fake_used() == before
+    """, """
+    others = [svo.ComputeManager(0) for _ in range(3)]
+    fake.fake_limit(fake.fake_used() + 90 * MiB)  # for two builds and a buffer at a time
+    failed = []
+    def work(c, k):
+        for _ in range(20):
+            try:
+                if k:
+                    c.BuildTreeDevice(geometry, 1, 4)
+                else:
+                    c.InitDeviceBuffer(B.OutputImage, 60 * MiB, 1)
+                    c.ReleaseBuffer(B.OutputImage)
+            except svo.SvoError as e:
+                if "out of memory" not in str(e): failed.append(e)  # both at once may not fit
+    threads = [threading.Thread(target=work, args=(c, k)) for k, c in enumerate(others)]
+    for t in threads: t.start()
+    for t in threads: t.join()
+    assert not failed, failed
+    fake.fake_limit(1 << 32)
+    for c in (cm, *others): c.Dispose()
+    assert fake.fake_used() == 0
+    """], ids=["same context", "another context", "too large", "release", "dispose", "threads"])
+def test_kept_build_memory_is_given_back(fake, code):
+    fake_hip.run(fake, textwrap.dedent(KEPT) + textwrap.dedent(code))
 
 
 @pytest.mark.gpu
