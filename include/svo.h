@@ -255,7 +255,9 @@ int svo_buffer_fill(svo_context *ctx, int buffer_name, const void *pattern, size
 /* Device-to-device copy between two named buffers (the clEnqueueCopyBuffer role; the reference's
  * ComputeManager has no counterpart).  Asynchronous on the context's stream. */
 int svo_buffer_copy(svo_context *ctx, int dst_name, size_t dst_offset, int src_name, size_t src_offset, size_t bytes);
-/* ResetIDBuffer, ComputeManager.cs:232-241: read a u32 counter, then set it to 0 (blocking). */
+/* ResetIDBuffer, ComputeManager.cs:232-241: read a u32 counter, then set it to 0 (blocking: what was
+ * enqueued on the context before is done when the call returns, and the counter is 0 for whatever
+ * is enqueued afterwards, on this or any other stream). */
 int svo_reset_id(svo_context *ctx, int buffer_name, uint32_t *count_out);
 /* ZeroIDBuffer, ComputeManager.cs:243-249. */
 int svo_zero_id(svo_context *ctx, int buffer_name);

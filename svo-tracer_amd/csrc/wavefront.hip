@@ -444,12 +444,13 @@ __global__ void __launch_bounds__(kThreads) append_kernel(AppendParams a, uint32
   }
 }
 
-// ResetIDBuffer's device half: the counter goes to pinned host memory, tagged with the call's
-// number, and is cleared.
+// ResetIDBuffer's device half: the counter is cleared and goes to pinned host memory, tagged with the
+// call's number.  The host returns on the word, without a wait for the stream, so the clear is
+// released to the system before it: no work enqueued afterwards, on any stream, sees the old value.
 __global__ void take_counter_kernel(uint32_t *counter, unsigned long long *host, uint32_t tag) {
   const uint32_t v = *counter;
   *counter = 0u;
-  __hip_atomic_store(host, ((unsigned long long)tag << 32) | v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  __hip_atomic_store(host, ((unsigned long long)tag << 32) | v, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 template <int KIND, class Params>
