@@ -107,5 +107,5 @@ def test_frame_after_a_refused_buffer(svo, gpu):
     spec = svo.scenes.sphere_noise_scene(seed=1, max_depth=5, base_depth=2)
     with pytest.raises(svo.SvoError):
         gpu.InitDeviceBuffer(B.PruningBlockData, 1 << 46, 16)
-    count, _ = gpu.BuildTreeDevice(spec.geometry, spec.base_depth, spec.max_depth)
+    count, _ = gpu.BuildTreeDevice(spec.geometry, spec.base_depth, spec.max_depth, spec.max_size)
     assert count == spec.build().block_count
