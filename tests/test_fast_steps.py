@@ -5,7 +5,9 @@ field, cones nearer than 2^-6 to the camera (the footprint's exact form), levels
 frames that refill lanes early."""
 from __future__ import annotations
 
+import hashlib
 import math
+from pathlib import Path
 
 import numpy as np
 import pytest
@@ -14,6 +16,7 @@ from frame_helpers import assert_frame_matches, gpu_frame, tree_arrays
 
 pytestmark = pytest.mark.gpu
 
+GOLDEN = Path(__file__).parent / "golden"
 IDENT = [1.0, 0.0, 0.0, 0.0, 1.0, 0.0, 0.0, 0.0, 1.0]
 
 
@@ -76,15 +79,55 @@ def test_cameras(svo, orc, gpu, name, refill):
 
 @pytest.mark.parametrize("name", NAMES + BEYOND_ORACLE)
 def test_both_forms_agree(svo, gpu, name):
-    """With early refills every step is a general one; otherwise ordinary cones take fast steps.
-    Stray cones (NaN, vanishing or huge directions), whose blocks are those they entered, are
-    compared between the two only: the oracle looks a block up by the location."""
+    """With early refills every step is a general one; otherwise ordinary cones take fast steps."""
     cam = dict(cameras(svo))[name]
     tree, bases, blocks = tree_arrays(svo, svo.scenes.config1_scene())
     a, b = (gpu_frame(svo, gpu, bases, blocks, tree.initial_usages(0), cam, refill_lanes=r) for r in (0, 24))
     for key in ("hit", "visits", "status", "hash", "depth", "location", "usages", "requests"):
         assert np.array_equal(a[key], b[key]), key
     assert np.array_equal(a["rgba"], b["rgba"]) and a["request_count"] == b["request_count"]
+
+
+def stray_outputs(svo, cm, name, **opts):
+    """A stray camera's outputs: hits and visits, and digests of the other arrays, of a frame, of one
+    with a stack of two levels (keys s2-) and of four composited layers (key layers)."""
+    cam = dict(cameras(svo))[name]
+    tree, bases, blocks = tree_arrays(svo, svo.scenes.config1_scene())
+
+    def digest(a):
+        return np.array(hashlib.sha256(np.ascontiguousarray(a).tobytes()).hexdigest())
+
+    out = {}
+    for prefix, extra in (("", {}), ("s2-", {"stack_levels": 2})):
+        o = gpu_frame(svo, cm, bases, blocks, tree.initial_usages(0), cam, **opts, **extra)
+        out[prefix + "hit"], out[prefix + "visits"] = o["hit"], o["visits"]
+        out[prefix + "request_count"] = np.array(o["request_count"])
+        for key in ("status", "hash", "depth", "location", "usages", "requests"):
+            out[prefix + key] = digest(o[key])
+        # (a NaN's bits are not the frame's to define)
+        out[prefix + "rgba"] = digest(np.where(np.isnan(o["rgba"]), np.float32(-1), o["rgba"]))
+    if not opts:
+        B, n = svo.BufferName, cam.screen_size[0] * cam.screen_size[1]
+        cm.InitBuffer(B.LeafParams, np.random.default_rng(4).random((blocks.size, 4), np.float32))
+        cm.InitDeviceBuffer(B.Layers, n, 16)
+        cm.Composite([cam], layers=True)
+        out["layers"] = digest(cm.ReadBuffer(B.Layers, np.uint32, 4 * n))
+        for buffer in (B.LeafParams, B.Layers):
+            cm.ReleaseBuffer(buffer)
+    return out
+
+
+@pytest.mark.parametrize("name", BEYOND_ORACLE)
+@pytest.mark.parametrize("refill", [0, 24])
+def test_stray_cones(svo, gpu, name, refill):
+    """Stray cones (NaN, vanishing or huge directions), whose blocks are those they entered while the
+    oracle looks a block up by the location, have the outputs of the kernel that knew one step form
+    only (tests/golden/make_stray_fixture.py)."""
+    want = np.load(GOLDEN / "stray_cones.npz")
+    got = stray_outputs(svo, gpu, name, **({"refill_lanes": refill} if refill else {}))
+    for key, value in got.items():
+        assert np.array_equal(value, want[f"{name}/{key}"]), key
+    assert (got["hit"] != 0xFFFFFFFF).any() or (got["visits"] > 0).any()
 
 
 def deep_chain(svo, levels: int, at):
