@@ -75,9 +75,10 @@ struct FrameParams {
   uint32_t ticked_slots;  // slots of the LDS table of ticked usage groups (0: no table)
   uint32_t refill;
   uint32_t lanes;  // lanes of a wave that take cones, a power of two (64: all)
-  uint32_t chunk;  // work items a wave claims per atomic (multiple of 64)
-  // tile schedule (may be null): position k of a band's work range holds tile order[k]; a
-  // wave stores the most steps any of a tile's cones took in tile_cost[tile]
+  uint32_t chunk;  // work items a wave claims per atomic: a multiple of 64, or `lanes`
+  // tile schedule (may be null): position k of a band's work range holds tile order[k]; the waves
+  // that run a tile, or a part of it each (lanes < 64), raise tile_cost[tile] from 0 to the most
+  // steps any of its cones took
   const uint32_t *order;
   uint32_t *tile_cost;
 };
@@ -124,7 +125,7 @@ struct FrameBegin {
   uint32_t bands;   // 0 (no tile order) or 8
   uint32_t stage;   // set by the launcher: stage the cost classes in LDS
   uint32_t n_views; // cameras of the frame (all inline when n_cams > 0)
-  const uint32_t *cost;
+  uint32_t *cost;   // cleared once the order has been made
   uint32_t *order;
   float *views;     // per band, n_views records of kViewWords floats
   uint32_t range_begin[9];

@@ -370,7 +370,7 @@ trace_frame_kernel(const FrameParams p) {
     if (p.tile_cost && cur_tile != kU32Max) {
       uint32_t a = nvis;
       for (int off = 32; off > 0; off >>= 1) a = max(a, (uint32_t)__shfl_xor((int)a, off));
-      if (lane == 0u) p.tile_cost[cur_tile] = a;
+      if (lane == 0u) atomicMax(&p.tile_cost[cur_tile], a);  // several waves may run a part of it each
     }
     cur_tile = kU32Max;
     if (!active) nvis = 0;
@@ -830,9 +830,9 @@ __device__ bool views_coherent(const CamRec *cams, uint32_t n, float *saved) {
 // The work a frame does before its trace launch, in one launch: work-group 0 clears the
 // frame's counters and totals and writes the camera records that came in the kernel
 // argument; work-group b < bands builds band b's tile order (cost order when the views
-// are coherent with the band's recorded ones, raster order otherwise).  The camera poses
-// are read from the argument when they came inline (work-group 0 may still be writing the
-// device records), from the device records otherwise (copied before this launch).
+// are coherent with the band's recorded ones, raster order otherwise) and clears its costs.  The
+// camera poses are read from the argument when they came inline (work-group 0 may still be
+// writing the device records), from the device records otherwise (copied before this launch).
 __global__ void __launch_bounds__(kOrderThreads) frame_begin_kernel(FrameBegin f) {
   if (blockIdx.x == 0) {
     const uint32_t i = threadIdx.x;
@@ -850,6 +850,8 @@ __global__ void __launch_bounds__(kOrderThreads) frame_begin_kernel(FrameBegin f
     } else {
       for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) f.order[b0 + i] = b0 + i;
     }
+    __syncthreads();  // the order has read the costs, which the frame's waves raise from 0
+    for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) f.cost[b0 + i] = 0u;
   }
 }
 

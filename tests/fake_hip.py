@@ -1,6 +1,6 @@
-"""Runs host code of the library on the CPU over fake_hip.cpp: a child process loads the fake
-runtime, then the library, and runs the code given (``svo``, ``fake``, ``B`` and ``cm``, a context,
-are there)."""
+"""Runs code in a child process with a library between libsvo and the HIP runtime: fake_hip.cpp in the
+runtime's place, for host code on the CPU, or launch_spy.cpp before it.  The child loads that library
+(``fake``), then libsvo, and runs the code given (``svo``, ``B`` and ``cm``, a context, are there)."""
 from __future__ import annotations
 
 import shutil
@@ -14,8 +14,9 @@ TESTS = Path(__file__).resolve().parent
 PRELUDE = f"""
 import ctypes, sys
 fake = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
-fake.fake_limit.argtypes = [ctypes.c_size_t]
-fake.fake_used.restype = fake.fake_launches.restype = ctypes.c_size_t
+if hasattr(fake, "fake_limit"):
+    fake.fake_limit.argtypes = [ctypes.c_size_t]
+    fake.fake_used.restype = fake.fake_launches.restype = ctypes.c_size_t
 sys.path.insert(0, {str(TESTS.parent / "svo-tracer_amd")!r})
 import _loader
 import numpy as np
@@ -25,11 +26,12 @@ MiB = 1 << 20
 """
 
 
-def build(folder: Path) -> Path:
-    lib = folder / "libfakehip.so"
+def build(folder: Path, name: str = "fake_hip") -> Path:
+    lib = folder / f"lib{name}.so"
     hip = Path(shutil.which("hipcc") or "/opt/rocm/bin/hipcc").resolve().parents[1]
     subprocess.run(["g++", "-std=c++17", "-O1", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__", f"-I{hip}/include",
-                    str(TESTS / "fake_hip.cpp"), "-o", str(lib)], check=True)
+                    f"-I{TESTS.parent / 'svo-tracer_amd' / 'csrc'}", f"-I{TESTS.parent / 'include'}",
+                    str(TESTS / f"{name}.cpp"), "-o", str(lib), "-ldl"], check=True)
     return lib
 
 
