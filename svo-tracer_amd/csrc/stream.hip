@@ -74,7 +74,8 @@ __device__ __forceinline__ uint32_t compact3(uint32_t v) {  // every third bit -
 }
 
 // Any builder geometry: one cell's classification and one block (MakeChunk / MakeBlock,
-// TreeBuilder.cs:74-93, 264-284), by the rules the host builder shares.
+// TreeBuilder.cs:74-93, 264-284), by the rules the host builder shares.  (The sphere + noise SDF is
+// classified eight cells at a time, in geom_chunk.)
 __device__ void geom_classify(const GeomView &g, uint32_t level, uint32_t x, uint32_t y, uint32_t z, bool *air,
                               bool *geo) {
   switch (g.kind) {
@@ -87,11 +88,8 @@ __device__ void geom_classify(const GeomView &g, uint32_t level, uint32_t x, uin
     case SVO_GEOMETRY_SPHERES:
       shapes::spheres_classify(g.shapes, g.count, shapes::cell_box(level, x, y, z), air, geo);
       return;
-    case SVO_GEOMETRY_CUBES:
-      shapes::cubes_classify(g.shapes, g.count, shapes::cell_box(level, x, y, z), air, geo);
-      return;
     default:
-      shapes::noise_classify(g.noise, level, x, y, z, air, geo);
+      shapes::cubes_classify(g.shapes, g.count, shapes::cell_box(level, x, y, z), air, geo);
   }
 }
 

@@ -85,7 +85,7 @@ struct FrameParams {
 
 struct LaunchShape {
   int workgroup;
-  int waves;  // register budget: waves per SIMD the kernel is compiled for (6)
+  int waves;  // register budget: waves per SIMD the kernel is compiled for (4..6)
   int grid;
   int max_grid;  // work-groups that can find work
   size_t lds_bytes;
