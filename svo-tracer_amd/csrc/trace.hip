@@ -25,10 +25,12 @@
 //     the high words of the location, the minor axes' moves as two float-to-u32 conversions
 //     without the saturation they cannot reach, the LOD tests through an approximate footprint
 //     checked against its error, blocks without their addresses on the stack, usage ticks where
-//     a block is entered instead of at every visit.  1080p depth-12 frame: 386.7 M -> 247.7 M
-//     VALU instructions, 0.639 -> 0.495 ms a frame with three frames in flight, 0.90 -> 0.65 ms
-//     alone; the 64-camera batch 8.11 -> 6.05 ms; forward + adjoint of 32 x 512^2 9.46 ->
-//     6.76 ms (there the outputs of ended cones also moved out of the step loop);
+//     a block is entered instead of at every visit.  1080p depth-12 frame: 386.7 M -> 244.4 M
+//     VALU instructions, 0.638 -> 0.484 ms a frame with three frames in flight, 0.87 -> 0.65 ms
+//     alone; the 64-camera batch 8.34 -> 6.10 ms (VALU busy 99 %); forward + adjoint of 32 x 512^2
+//     9.45 -> 6.75 ms (there the outputs of ended cones also moved out of the step loop).  Frames
+//     that keep the general form gained from the rest: with depth of field 0.81 -> 0.72 ms alone,
+//     with lanes refilled from 32 idle ones on 1.05 -> 0.90 ms;
 //   - per-cone outputs are written by cone id; queue order is made canonical
 //     (ascending cone id) by the order-preserving compaction kernels below.
 #include <hip/hip_runtime.h>

@@ -12,7 +12,8 @@
 // loop is some 770 steps, most of a few thousand items at its end, so a step is bound by its
 // launches: one or two instead of four, with coalesced appends (a thread that walked 16
 // consecutive items took 12.9 us a launch), made the appends of the 1080p depth-12 loop
-// 15.3 -> 1.7 ms of kernel time a frame and the frame 27 -> 18 ms (the host calls included).
+// 15.3 -> 1.7 ms of kernel time a frame and, with the counter read-backs below, the frame 28.4 ->
+// 15.6 ms (the host calls included).
 #include <hip/hip_runtime.h>
 
 #include "svo_device.hpp"
